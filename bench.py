@@ -658,6 +658,8 @@ def main():
     if pt64 is None:  # no pass launch in the timed region (one iteration per launch): the region itself
         pt64 = {"iters_per_launch": 1, "launches": a.steps, "launch_s": gpu_s / a.steps}
     k_pass = pt64["iters_per_launch"]
+    for k in (5, 6, 7):  # the size default's passes: pipelined on large grids, resident on small ones
+        names[k] = (f"ptp_tile_f64<{k}>" if nx >= 800 else "ptr_tile_f64", f"ptp{k}_tile_f64")
     kernel, prof = names[k_pass]
     line = {
         "metric": "PT iters/s + T_eff HBM GB/s; time-to-1e-8 FP32-refined vs FP64; batched solves/s",

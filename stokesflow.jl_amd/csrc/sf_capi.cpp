@@ -167,7 +167,7 @@ int PTLoop::pair(hipStream_t s, int k)
         const int r = tm->begin(s, 0, k);
         if (r) return r;
     }
-    const hipError_t e = launch_pt_multi(pp, k, s);
+    const hipError_t e = plan.kind != PT_PLAN_NONE ? launch_pt_plan(pp, plan, k, s) : launch_pt_multi(pp, k, s);
     pp.seg = seg1;  // the one-iteration kernel keeps its own tile rows
     HIPCHK(e);
     if (tm && tm->on) {
@@ -211,6 +211,10 @@ int PTLoop::run_fixed(int64_t n_iter, hipStream_t s)
 {
     int64_t it = 0;
     int rc = SF_OK;
+    // A pipelined run of less than two whole passes keeps the one-wave passes of up to four
+    // iterations, the launch plan that the pass timer has reported for such runs.
+    int kmax = this->kmax;
+    if (plan.kind == PT_PLAN_PIPE && n_iter < 2 * kmax) kmax = 4;
     for (int k = kmax; pairs && k >= 2; --k)
         for (; it + k <= n_iter && rc == SF_OK; it += k) rc = pair(s, k);
     for (; it < n_iter && rc == SF_OK; ++it) rc = single(0, s);
@@ -773,6 +777,7 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
     };
     sf_pt_tuning bestv{}, best_all{};
     bestv.us_per_iter = 1e300;
+    double plan_us = 1e300;
     // first the shapes of the one-iteration kernel; every loop ends at the first error
     const int rc = [&]() -> int {
         c->fuse64 = 1;
@@ -810,7 +815,14 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
                 if (t.us_per_iter < best_all.us_per_iter) best_all = t;
             }
         }
-        return SF_OK;
+        // last the size default's pass, which is kept where none of the table is faster
+        const int explicit_fuse = c->fuse, explicit_rows = c->pair_rows;
+        c->fuse64 = c->rows64 = c->fuse = c->pair_rows = 0;
+        const int n_plan = std::max(28, (iters + 27) / 28 * 28);
+        const int r = time_shape(PT_PLAN_MAX_K, n_plan, &plan_us);
+        c->fuse = explicit_fuse;
+        c->pair_rows = explicit_rows;
+        return r;
     }();
     (void)hipStreamSynchronize(s);
     release();
@@ -828,6 +840,7 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
     // the FP64 passes only: the FP32 sweeps of the refined solver keep their own defaults
     c->fuse64 = best_all.iters_per_launch;
     c->rows64 = best_all.iters_per_launch > 1 ? best_all.rows : 0;
+    if (plan_us < best_all.us_per_iter) c->fuse64 = c->rows64 = 0;
     if (best) *best = best_all;
     if (n_table) *n_table = nt;
     return SF_OK;

@@ -155,11 +155,13 @@ struct PTLoop {
     double *vx0, *vy0, *p0, *dvx0, *dvy0;  // the caller's arrays
     PTBuffers b;
     bool pairs;  // multi-iteration passes enabled (b.dvx_b, b.dvy_b must then be set)
-    int kmax;    // iterations per pass (2, 3 or 4)
-    int rows;    // tile rows of the passes (0: size default)
+    int kmax;    // iterations per pass (2 to 4; to 7 with a plan)
+    int rows;    // tile rows of the one-wave passes (0: size default)
+    PTPlan plan; // the size default's pass (kind PT_PLAN_NONE: an explicit setting's one-wave passes)
     PassTimer* tm = nullptr;  // times the pass launches when set and on
 
-    // fuse: iterations per pass (0 size default, 1 one per launch, 2 to 4; larger values cap at 4)
+    // fuse: iterations per pass (0 size default, 1 one per launch, 2 to 4; larger values cap at 4);
+    // pass_rows > 0 asks for the one-wave passes with that tile height
     void init(const PTBuffers& buf, int fuse, int pass_rows, int nx_, int ny_, double* Vx_s, double* Vy_s, double* P,
               double* dVx, double* dVy)
     {
@@ -179,6 +181,11 @@ struct PTLoop {
         rows = pass_rows;
         pairs = fuse != 1;
         kmax = fuse == 0 ? pt_default_fusion(nx, ny) : std::min(fuse, 4);
+        plan = PTPlan{};
+        if (fuse == 0 && pass_rows == 0) {
+            plan = pt_plan(nx, ny);
+            kmax = plan.k;
+        }
     }
     // One iteration (flags: check-iteration outputs); dV in place.
     int single(int flags, hipStream_t s);

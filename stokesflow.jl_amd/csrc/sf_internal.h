@@ -78,9 +78,25 @@ int pt2_default_rows(int nx, int ny);
 hipError_t launch_pt_multi(const PTParams& p, int k, hipStream_t s);
 // tile height of a k-iteration pass (k >= 3) when `copies` grids of this size share the launch
 int ptk_default_rows(int k, int nx, int ny, int copies = 1);
+// k = 5, 6 or 7 PT iterations per pass, pipelined over the waves of a workgroup (sf_ptp_tile.h), in
+// tiles of `rows` rows.
+hipError_t launch_pt_pipe(const PTParams& p, int k, int rows, hipStream_t s);
+// k PT iterations per pass on tiles of waves * r rows held in registers (sf_ptr_tile.h).
+#define PTR_MAX_NODES ((int64_t)1 << 28)
+hipError_t launch_pt_resident(const PTParams& p, int k, int r, int waves, hipStream_t s);
+// The size default: which of the two a grid takes, with what shape, and up to how many iterations
+// per pass; launch_pt_plan runs a pass of 2 <= k <= plan.k iterations.
+enum { PT_PLAN_NONE = 0, PT_PLAN_RESIDENT = 1, PT_PLAN_PIPE = 2, PT_PLAN_MAX_K = 7 };
+struct PTPlan {
+    int kind, k;
+    int rows;      // pipelined: rows per tile
+    int r, waves;  // resident: rows per wave, waves
+};
+PTPlan pt_plan(int nx, int ny);
+hipError_t launch_pt_plan(const PTParams& p, const PTPlan& plan, int k, hipStream_t s);
 // Snapshot staging: dst = (float)(src + shift) (sf_snapshot.hip).
 hipError_t launch_snap_cast(const double* src, float* dst, int64_t n, double shift, hipStream_t s);
-int pt_default_fusion(int nx, int ny);  // iterations per pass when the context leaves it open
+int pt_default_fusion(int nx, int ny);  // one-wave iterations per pass when only the tile rows are given
 int corr_default_fusion(int nx, int ny);  // FP32 correction sweeps per pass, likewise
 hipError_t launch_pt_resid_y(const ResYParams& p, hipStream_t s);
 hipError_t launch_reduce(const RedParams& p, int narr, int nb, hipStream_t s);

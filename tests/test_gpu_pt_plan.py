@@ -1,0 +1,48 @@
+"""The size defaults' passes (tiles held in registers, tiles pipelined over a workgroup's waves)
+against the CPU oracle, bit for bit, at the edges of their strips and tiles."""
+import numpy as np
+import pytest
+import torch
+
+import sfhip
+from oracle import sf_oracle as O
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+STATE = ("P", "Vx_s", "Vy_s", "dVx", "dVy")
+
+
+def _compare(S, nx, ny, n_iter):
+    args = (1.3, 0.9 / (nx - 1), 1.1 / (ny - 1))
+    G = {k: sfhip.from_numpy(S[k]) for k in STATE + ("rho_vy", "mu_b", "mu_p")}
+    sfhip.set_pt_fusion(nx, ny, 0, 0)
+    sfhip.pt_iterations(n_iter, G["P"], G["Vx_s"], G["Vy_s"], G["dVx"], G["dVy"], G["rho_vy"], G["mu_b"], G["mu_p"],
+                        *args, nx, ny, 0.01)
+    torch.cuda.synchronize()
+    O.compute_timesteps(S, nx, ny, *args[1:])
+    O.pt_iterations(S, nx, ny, n_iter, *args, 0.01)
+    for k in STATE:
+        assert np.array_equal(sfhip.to_numpy(G[k]), S[k], equal_nan=True), (nx, ny, n_iter, k)
+
+
+# grids of one strip and one tile, one column or row past it, several rows per wave, and (from 745
+# nodes per side) the pipelined pass with tiles that end on, before and after the last row
+@pytest.mark.parametrize("nx,ny", [(3, 3), (4, 17), (50, 4), (51, 5), (52, 9), (101, 64), (103, 131), (301, 257), (450, 449),
+                                   (640, 333), (760, 745), (801, 800), (1001, 777), (2301, 401)])
+def test_size_default_passes_bitwise(gpu, nx, ny):
+    n_iter = 2 * 7 + 6 + 1 if nx >= 700 else 41  # whole passes and a remainder
+    _compare(cases.random_state(nx, ny, seed=nx * 13 + ny), nx, ny, n_iter)
+
+
+@pytest.mark.parametrize("nx,ny", [(70, 40), (770, 760)])
+@pytest.mark.parametrize("log2_mu", [-260, 260])
+def test_size_default_passes_extreme_viscosity(gpu, nx, ny, log2_mu):
+    """Rows whose viscosity leaves the range of the short division sequence take the full one (the
+    scheme overflows with 2^-260: infinities and NaN then stand where the oracle has them)."""
+    S = cases.random_state(nx, ny, seed=5)
+    S["mu_p"][:, ny // 3: ny // 2] *= 2.0 ** log2_mu
+    for k in STATE:
+        S[k][:] = 0.0
+    _compare(S, nx, ny, 15)
