@@ -276,25 +276,19 @@ hipError_t launch_batch_solve(const BatchInstance* inst, const int* order, int n
 int batch_blocks_per_cu(int threads);
 
 // ---- marker -> grid ----
-// One marker's contribution in cell order: the relative position in its cell, its value and
-// its index (the merge key).  32 bytes, so a merge step reads one record from one cache line.
-struct M2GRec {
-    double dx, dy, val;
-    int idx, pad;
-};
-
+#define M2G_SPREAD 4112
 struct M2GScratch {
     int64_t cap_markers = 0;
     int64_t cap_cells = 0;
     int* key = nullptr;      // [nm] cell key or -1
+    int* loc = nullptr;      // [nm] place in the cell; after the scatter, two lists of tiles and parts
     int* count = nullptr;    // [cells]
     int* offset = nullptr;   // [cells + 1]
-    int* fill = nullptr;     // [cells]
     int* rec_idx = nullptr;  // [nm] marker index in cell order
-    M2GRec* rec = nullptr;   // [nm] records in cell order
     int* blocksums = nullptr;  // scan scratch
     int64_t cap_blocks = 0;
-    unsigned long long* counters = nullptr;  // [4]: bad, empty, nonfinite, spare
+    unsigned long long* counters = nullptr;  // [4]: bad, empty, nonfinite, listed tiles
+    unsigned long long* spread = nullptr;    // [M2G_SPREAD] listed parts, counters of empty nodes
 };
 
 hipError_t m2g_run(M2GScratch& s, double xmin, double ymin, double* val_grid, int gnx, int gny, const double* x_m,

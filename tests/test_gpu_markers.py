@@ -60,6 +60,37 @@ def test_m2g_bitwise_vs_oracle(gpu, origin, nx, ny, md, seed):
     assert nb >= 2
 
 
+@pytest.mark.parametrize("nx,ny,nm,cluster", [
+    (2, 2, 1, None),            # one marker
+    (17, 25, 300, None),        # under a marker per cell: the highest tiles, one row and column left over
+    (16, 22, 5600, None),       # whole tiles
+    (33, 9, 21000, None),       # the densest tiles: many columns are too long for one
+    (18, 11, 20000, None),      # above: all from global memory
+    (40, 37, 24000, 0.3),       # tiles that fit in parts only
+    (40, 37, 24000, 0.08),      # parts that do not fit either
+    (9, 8, 9000, 0.01),         # one cell with several sorted runs
+])
+def test_m2g_tile_forms_bitwise_vs_oracle(gpu, nx, ny, nm, cluster):
+    rng = np.random.default_rng(nx * 1000 + nm)
+    dx, dy = 1.0 / (nx - 1), 0.7 / (ny - 1)
+    x, y = rng.random(nm), 0.7 * rng.random(nm)
+    if cluster:
+        k = nm // 2  # in random order, as the rest
+        x[:k] = 0.41 + cluster * (rng.random(k) - 0.5)
+        y[:k] = 0.33 + cluster * (rng.random(k) - 0.5)
+        perm = rng.permutation(nm)
+        x, y = x[perm], y[perm]
+    val = 1.0 + rng.random(nm)
+    grid0 = np.asfortranarray(rng.random((nx, ny)))
+    vg, (vws, ws), st = m2g_gpu(0.0, 0.0, grid0, x, y, val, dx, dy, helper_shape=(nx, ny), helper_fill=3.0)
+    eg = grid0.copy(order="F")
+    evws, ews = O.zeros(nx, ny), O.zeros(nx, ny)
+    nb, ne = O.marker_to_grid(0.0, 0.0, eg, x, y, val, dx, dy, evws, ews)
+    assert np.array_equal(vg, eg)
+    assert np.array_equal(vws, evws) and np.array_equal(ws, ews)
+    assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
+
+
 def test_m2g_empty_nodes_keep_old_values(gpu):
     grid0 = np.asfortranarray(np.arange(20.0).reshape(4, 5, order="F"))
     x = np.array([0.01, 0.02])
