@@ -229,9 +229,9 @@ int sf_solve_stokes_refined(sf_ctx *ctx, double *P, double *Vx_pad, double *Vy_p
  * sets fit budget_mb; each instance is checked at its own ncheck iterations and retired on
  * convergence, and the set is refilled from the largest-first queue.
  * GRID: the instances one after another, each solved by ONE launch that spans the chip (at most
- * one workgroup of one to eight waves per CU): the whole PT loop with its checks, dt refreshes
- * and convergence test runs on the device, the passes (up to three PT iterations each, or
- * prm->depth) separated by a grid barrier; no host synchronisation, so it can be captured
+ * one workgroup per CU): the whole PT loop with its checks, dt refreshes and convergence test
+ * runs on the device, the passes (of as many PT iterations as pays at the size, or prm->depth)
+ * separated by a grid barrier; no host synchronisation, so it can be captured
  * (sf_graph_*).  A barrier wait longer than the limit (5 s unless sf_set_grid_wait_limit sets
  * another; workgroups not all resident) ends the launch and the call returns SF_ERR_HIP.
  * With precision 1 (WIDE only) every instance is solved as sf_solve_stokes_refined solves it,
@@ -253,7 +253,7 @@ enum { SF_BATCH_AUTO = 0, SF_BATCH_PERSISTENT = 1, SF_BATCH_WIDE = 2, SF_BATCH_G
 typedef struct {
     int rows;         /* grid rows per tile (<= 0: per instance, as the single solver's default) */
     int depth;        /* wide: rows of operands prefetched, 1 or 2 (<= 0: 1); grid: PT iterations per
-                         pass, 1 to 3 (<= 0: 3) */
+                         pass, 1 to 3 (<= 0: by size) */
     int threads;      /* persistent: threads per instance workgroup, multiple of 64, <= 512 (<= 0: 512) */
     int max_blocks;   /* persistent: cap on concurrently resident instances (<= 0: as many as fit) */
     int mode;         /* SF_BATCH_*; AUTO = WIDE */
@@ -380,7 +380,7 @@ int sf_ensemble_destroy(sf_ensemble *ens);
  * solve runs in the GRID mode of sf_solve_stokes_batched (one launch over the whole chip with the
  * PT loop, its checks and its convergence test on the device), and RK4 reads the new dt on the
  * device, so sf_graph_step replays n_steps timesteps with no host synchronisation in between.
- * args as for sf_step (its dt is the first step's input dt); iters_per_pass 1 to 3 (0: 3).
+ * args as for sf_step (its dt is the first step's input dt); iters_per_pass 1 to 3 (0: by size).
  * Fields, markers and dt are bit-identical to n_steps sf_step calls; err agrees to rounding
  * (its sum runs in another order).  The arrays must outlive the graph; it runs on a stream of its
  * own, ordered after the context's stream at each call, and sf_graph_step returns once the steps

@@ -8,6 +8,15 @@ using namespace sf;
 
 namespace sf {
 
+// Grid mode: what a pass costs besides its iterations, us: the barrier, and the tile read again past
+// caches that the barrier has emptied.  (384x300 takes 2.58 us per iteration planned with 4, 2.46 with 8;
+// 97x130 2.04 with 8, 2.10 with 11.)
+#define GRID_PASS_US 8.0
+// and the grids that resident passes are for: 1000x777 takes 7.7 us per iteration with them and 9.6
+// with one-wave passes of three, 1024^2 11.3 and 10.9, larger ones the same within 7% (64^2 1.83 and 3.48,
+// 301x257 2.34 and 4.09, 512^2 3.55 and 8.04).
+#define GRID_RESIDENT_NODES 900000
+
 // Per-instance scratch (doubles) of the batched solver: ping-pong state, tau/divV, Rx/Ry, scalars.
 size_t batch_scratch_doubles(int nx_, int ny_)
 {
@@ -202,10 +211,22 @@ BatchShape grid_shape(int nx, int ny)
     return sh;
 }
 
-// Grid mode: the launch of an instance, one wave per tile of its largest pass spread one wave per
-// CU first, then up to GRID_WG_WAVES waves per workgroup (at most one workgroup per CU).
+// Grid mode: the launch of an instance.  k = 0: resident passes up to GRID_RESIDENT_NODES.
+// One-wave passes of k iterations: a wave per tile of the largest pass, spread one wave per CU first,
+// then up to GRID_WG_WAVES waves per workgroup.  At most one workgroup per CU either way.
 GridShape grid_launch_shape(const BatchInstance& d, int k)
 {
+    if (k == 0) {
+        double us;
+        const PTPlan plan = pt_plan_resident(d.nx, d.ny, GRID_RESIDENT_MAX_K, GRID_PASS_US, &us);
+        if (plan.kind == PT_PLAN_RESIDENT && (int64_t)d.nx * d.ny <= GRID_RESIDENT_NODES) {
+            const int out = 64 - 2 * plan.k, seg = plan.waves * plan.r - 2 * plan.k;
+            const int64_t t = (int64_t)((d.nx - 1 + out - 1) / out) * ((d.ny + seg - 1) / seg);
+            const int nwg = (int)std::min<int64_t>(t, grid_capacity(plan.k, plan.r, plan.waves));
+            if (nwg > 0) return GridShape{nwg, plan.waves, plan.k, plan.r};
+        }
+        k = 3;
+    }
     int t = d.wpt[0].ntiles;
     if (k >= 2) t = std::max(t, d.wpt[2 * k - 2].ntiles);
     int cus = 256;
@@ -214,8 +235,8 @@ GridShape grid_launch_shape(const BatchInstance& d, int k)
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
         cus = 256;
     const int waves = std::max(1, std::min((t + cus - 1) / cus, (int)GRID_WG_WAVES));
-    const int nwg = std::max(1, std::min((t + waves - 1) / waves, grid_capacity(k, waves)));
-    return GridShape{nwg, waves};
+    const int nwg = std::max(1, std::min((t + waves - 1) / waves, grid_capacity(k, 0, waves)));
+    return GridShape{nwg, waves, k, 0};
 }
 
 }  // namespace sf
@@ -1045,7 +1066,7 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         // one instance after another, each solved by one launch over the whole chip
         rc = grid_reserve(c, n);
         if (rc) return rc;
-        const int k = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 3;
+        const int k = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 0;
         HIPCHK(hipMemsetAsync(c->g_sync, 0, sizeof(unsigned long long) * GRID_SYNC_WORDS * (size_t)n, s));
         const double wait_s = grid_wait_seconds();
         const uint64_t wait_ticks = grid_wait_limit();
@@ -1053,8 +1074,8 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
             const int i = order[(size_t)qi];
             const GridShape gs = grid_launch_shape(host[(size_t)i], k);
             const GridArgs ga{c->b_inst + i, c->b_res + i, c->g_sync + (size_t)GRID_SYNC_WORDS * i, c->g_part,
-                              gs.nwg, gs.waves, wait_ticks};
-            HIPCHK(launch_grid_solve(ga, k, s));
+                              gs.nwg, gs.waves, gs.k, gs.r, wait_ticks};
+            HIPCHK(launch_grid_solve(ga, s));
         }
         std::vector<unsigned long long> sync((size_t)GRID_SYNC_WORDS * n);
         HIPCHK(hipMemcpyAsync(res.data(), c->b_res, sizeof(BatchResult) * (size_t)n, hipMemcpyDeviceToHost, s));

@@ -11,7 +11,7 @@ struct sf_ensemble {
     hipStream_t stream = nullptr;  // own non-blocking stream: capture needs one
     hipEvent_t ev = nullptr;
     int n = 0, threads = 512, nblocks = 0, use_graph = 1, wide = 1, depth = 1;
-    int grid = 0, gk = 3;  // grid mode: one chip-wide launch per member, gk PT iterations per pass
+    int grid = 0, gk = 0;  // grid mode: one chip-wide launch per member, gk PT iterations per pass (0: by size)
     double budget = 0.0;
     std::vector<sf_step_args> mem;
     std::vector<sf_batch_instance> bi;     // the members as batched-solver instances (dt updated per step)
@@ -125,8 +125,8 @@ static hipError_t ensemble_enqueue_persistent(sf_ensemble* e)
             const int i = e->order[(size_t)q];
             const GridShape& gs = e->gshape[(size_t)i];
             const GridArgs ga{e->inst + i, e->res + i, e->gsync + (size_t)GRID_SYNC_WORDS * i, e->gpart, gs.nwg, gs.waves,
-                              grid_wait_limit()};
-            r = launch_grid_solve(ga, e->gk, e->stream);
+                              gs.k, gs.r, grid_wait_limit()};
+            r = launch_grid_solve(ga, e->stream);
         }
     } else {
         r = launch_batch_solve(e->inst, e->order_dev, e->n, e->queue, e->res, e->threads, e->nblocks, e->stream);
@@ -211,7 +211,7 @@ extern "C" int sf_ensemble_create(sf_ctx* c, const sf_step_args* members, int n,
     e->use_graph = use_graph ? 1 : 0;
     e->wide = (mode != SF_BATCH_PERSISTENT && mode != SF_BATCH_GRID);
     e->grid = (mode == SF_BATCH_GRID);
-    e->gk = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 3;
+    e->gk = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 0;
     e->refined = prm ? prm->precision : 0;
     if (e->refined != 0 && (e->refined != 1 || !e->wide)) {
         free_ensemble(e);

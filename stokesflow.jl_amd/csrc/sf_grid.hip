@@ -2,14 +2,17 @@
 //
 // solveStokes! (StokesSolver_multixpu.jl:43-95) has a data-dependent loop (convergence is tested
 // every ncheck iterations), which a hipGraph cannot hold.  Here the loop runs on the device: a
-// launch of at most one workgroup per CU, of one to eight waves, walks the same pass schedule as
-// sf_solve_stokes (passes of up to three PT iterations, the single iterations at checks, dt
-// refreshes and iterMax), each wave taking tiles t = band, band + G, ... of every pass (the waves
-// of one XCD hold consecutive bands), and a grid barrier separates the passes.  Small grids get one wave per CU (a wave alone on a SIMD runs its
-// tile faster), larger ones up to eight (fewer tiles per wave).  The dt refresh and the err check
+// launch of at most one workgroup per CU walks the same pass schedule as sf_solve_stokes (passes of
+// several PT iterations, the single iterations at checks, dt refreshes and iterMax), and a grid barrier
+// separates the passes.  Small and middle grids take passes of up to GRID_RESIDENT_MAX_K iterations on
+// tiles in registers, a tile per workgroup of up to 16 waves: the barrier, and the tile that every pass
+// reads past caches the barrier has emptied, cost about 8 us and are paid once per 5 to 14 iterations
+// (384x300: 2.46 us per iteration; 6.5 with passes of three).  Larger grids take passes of up to three on
+// tiles of one wave, one to eight waves per workgroup.  Tiles go out t = band, band + G, ... (the
+// workgroups of one XCD hold consecutive bands).  The dt refresh and the err check
 // reduce over the whole grid in two steps (a partial per wave, then every wave sums the partials
 // in the same order, so every wave takes the same decision).  Each tile is the code of the single
-// solver's pass kernels (sf_pt_tile.h, sf_pt2_tile.h, sf_ptk_tile.h), so every field is
+// solver's pass kernels (sf_pt_tile.h, sf_pt2_tile.h, sf_ptk_tile.h, sf_ptr_tile.h), so every field is
 // bit-identical to sf_solve_stokes; err is a sum of the same terms in another order (equal to
 // rounding).
 //
@@ -29,6 +32,7 @@
 #include <atomic>
 
 #include "sf_ptk_tile.h"
+#include "sf_ptr_tile.h"
 
 namespace sf {
 
@@ -209,9 +213,11 @@ __device__ inline void grid_copy(double* __restrict__ dst, const double* __restr
 
 }  // namespace
 
-// K = PT iterations per pass, 1 to 3 (the four-iteration tile spills beside the loop control).
-template <int K>
-__global__ __launch_bounds__(64 * GRID_WG_WAVES) void grid_solve_kernel(GridArgs a)
+// R = 0: one-wave passes of K iterations, 1 to 3 (the four-iteration tile spills beside the loop
+// control).  R > 0: passes of up to K = a.k iterations on tiles of R rows per wave held in registers, a
+// workgroup per tile.
+template <int K, int R>
+__global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) void grid_solve_kernel(GridArgs a)
 {
     CGrid& I = *(CGrid*)a.desc;
     // w is uniform in the wave (saying so keeps the tile indices in scalar registers)
@@ -257,35 +263,51 @@ __global__ __launch_bounds__(64 * GRID_WG_WAVES) void grid_solve_kernel(GridArgs
         return true;
     };
 
+    __shared__ double lds[R ? PTR_LDS(GRID_RESIDENT_WAVES) : 1];
+    const int band = __builtin_amdgcn_readfirstlane(bar.band), waves = blockDim.x >> 6;
     double err = 2.0 * eps;
     int64_t iter = 1;
     int pf = 0;  // passes so far, mod 2: the state (V, P, dV) is in the caller's buffers when 0
     while (err > eps && iter <= iter_max) {
-        // iterations iter..iter+K-1 in one pass when none is a check iteration, none but the last
-        // is followed by a dt refresh and the last is not iter_max (the rule of sf_solve_stokes;
-        // where K do not fit, single iterations follow, which gives the same bits)
-        bool fused = K > 1 && iter + K - 1 < iter_max;
-        for (int64_t j = iter; fused && j < iter + K; ++j) {
-            if (j % ncheck == 0) fused = false;
-            if (j < iter + K - 1 && fss && j % ndtupdate == 0) fused = false;
+        // iterations iter..iter+k-1 in one pass when none is a check iteration, none but the last
+        // is followed by a dt refresh and the last is not iter_max (the rule of sf_solve_stokes);
+        // one-wave passes have k = K, and where K do not fit, single iterations follow (the same
+        // bits); resident passes take as many as fit
+        int k = K;
+        if constexpr (R > 0) {
+            int64_t fit = ncheck - 1 - (iter - 1) % ncheck;
+            if (fss) fit = min(fit, ndtupdate - (iter - 1) % ndtupdate);
+            k = (int)min((int64_t)a.k, min(fit, iter_max - iter));
         }
+        bool fused = R > 0 ? k > 0 : K > 1 && iter + K - 1 < iter_max;
+        if constexpr (R == 0)
+            for (int64_t j = iter; fused && j < iter + K; ++j) {
+                if (j % ncheck == 0) fused = false;
+                if (j < iter + K - 1 && fss && j % ndtupdate == 0) fused = false;
+            }
         if (fused) {
-            const PTParams GRID_CONST& pp = I.wpt[2 * K - 2 + pf];
-            const int ntiles = pp.ntiles, nstrips = pp.nstrips;
-            if constexpr (K == 3) {
-                for (int t = wt; t < ntiles; t += nw) ptk_tile<3, 0>(pp, t % nstrips, t / nstrips);
-            } else if constexpr (K == 2) {
-                for (int t = wt; t < ntiles; t += nw) pt2_tile(pp, t % nstrips, t / nstrips);
+            const PTParams GRID_CONST& pp = I.wpt[(R > 0 ? 0 : 2 * K - 2) + pf];
+            if constexpr (R > 0) {
+                const int out = SF_WAVE - 2 * k, seg = waves * R - 2 * k;
+                const int nstrips = (nx - 1 + out - 1) / out, ntiles = nstrips * ((ny + seg - 1) / seg);
+                for (int t = band; t < ntiles; t += gridDim.x) ptr_tile<R>(pp, k, seg, t % nstrips, t / nstrips, lds);
+            } else {
+                const int ntiles = pp.ntiles, nstrips = pp.nstrips;
+                if constexpr (K == 3) {
+                    for (int t = wt; t < ntiles; t += nw) ptk_tile<3, 0>(pp, t % nstrips, t / nstrips);
+                } else if constexpr (K == 2) {
+                    for (int t = wt; t < ntiles; t += nw) pt2_tile(pp, t % nstrips, t / nstrips);
+                }
             }
             pf ^= 1;
             if (!bar.sync()) return;
-            if (fss && (iter + K - 1) % ndtupdate == 0) {
+            if (fss && (iter + k - 1) % ndtupdate == 0) {
                 double dtc;
                 if (!grid_dt(pp.vx_b, pp.vy_b, &dtc)) return;
                 if (blockIdx.x == 0 && threadIdx.x == 0) I.scal[SC_DT] = dtc;
                 if (!bar.sync()) return;
             }
-            iter += K;
+            iter += k;
             continue;
         }
         const PTParams GRID_CONST& pp = I.wpt[pf];
@@ -360,12 +382,12 @@ __global__ __launch_bounds__(64 * GRID_WG_WAVES) void grid_solve_kernel(GridArgs
     double dt_new;
     if (!grid_dt(Vx_s, Vy_s, &dt_new)) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        BatchResult* R = a.res;
-        R->dt_new = dt_new;
-        R->err = err;
-        R->niter = niter;
-        R->converged = err <= eps;
-        R->dt_last = I.scal[SC_DT];
+        BatchResult* res = a.res;
+        res->dt_new = dt_new;
+        res->err = err;
+        res->niter = niter;
+        res->converged = err <= eps;
+        res->dt_last = I.scal[SC_DT];
     }
 }
 
@@ -376,25 +398,35 @@ __global__ void grid_zero_sync(unsigned long long* p)
         if (k != GRID_SYNC_STICKY) p[k] = 0ull;
 }
 
-// Resident workgroups of `waves` waves of grid_solve_kernel<k> on the current device, at most
-// one per CU.
-int grid_capacity(int k, int waves)
+static const void* grid_kernel(int k, int r)
 {
-    static int cap[4][GRID_WG_WAVES + 1] = {};
-    if (k < 1 || k > 3 || waves < 1 || waves > GRID_WG_WAVES) return 0;
-    if (cap[k][waves] == 0) {
+    switch (r) {
+        case 0: return k == 3 ? (const void*)grid_solve_kernel<3, 0>
+                              : (k == 2 ? (const void*)grid_solve_kernel<2, 0> : (const void*)grid_solve_kernel<1, 0>);
+        case 1: return (const void*)grid_solve_kernel<0, 1>;
+        case 2: return (const void*)grid_solve_kernel<0, 2>;
+        default: return (const void*)grid_solve_kernel<0, 3>;
+    }
+}
+
+// Resident workgroups of `waves` waves of the kernel of (k, r) on the current device, at most one per CU.
+int grid_capacity(int k, int r, int waves)
+{
+    static int cap[7][GRID_RESIDENT_WAVES + 1] = {};
+    const int form = r ? 3 + r : k;
+    if (k < 1 || r < 0 || r > 3 || waves < 1) return 0;
+    if (r ? waves > GRID_RESIDENT_WAVES || k > GRID_RESIDENT_MAX_K || waves * r <= 2 * k : waves > GRID_WG_WAVES || k > 3) return 0;
+    if (cap[form][waves] == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             cus = 256;
-        const void* f = k == 3 ? (const void*)grid_solve_kernel<3>
-                               : (k == 2 ? (const void*)grid_solve_kernel<2> : (const void*)grid_solve_kernel<1>);
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 64 * waves, 0) != hipSuccess || per_cu < 1)
-            cap[k][waves] = -1;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grid_kernel(k, r), 64 * waves, 0) != hipSuccess || per_cu < 1)
+            cap[form][waves] = -1;
         else
-            cap[k][waves] = cus;
+            cap[form][waves] = cus;
     }
-    return std::max(cap[k][waves], 0);
+    return std::max(cap[form][waves], 0);
 }
 
 static std::atomic<double> grid_wait_s{(double)GRID_WAIT_SECONDS};
@@ -415,15 +447,13 @@ uint64_t grid_wait_limit()
 void grid_set_wait_seconds(double seconds) { grid_wait_s.store(seconds); }
 double grid_wait_seconds() { return grid_wait_s.load(); }
 
-hipError_t launch_grid_solve(const GridArgs& a, int k, hipStream_t s)
+hipError_t launch_grid_solve(const GridArgs& a, hipStream_t s)
 {
-    if (a.nwg < 1 || a.nwg > grid_capacity(k, a.wg_waves)) return hipErrorInvalidValue;
+    if (a.nwg < 1 || a.nwg > grid_capacity(a.k, a.r, a.wg_waves)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(grid_zero_sync, dim3(1), dim3(256), 0, s, a.sync);
-    const dim3 g(a.nwg), b(64 * a.wg_waves);
-    if (k == 3) hipLaunchKernelGGL(grid_solve_kernel<3>, g, b, 0, s, a);
-    else if (k == 2) hipLaunchKernelGGL(grid_solve_kernel<2>, g, b, 0, s, a);
-    else hipLaunchKernelGGL(grid_solve_kernel<1>, g, b, 0, s, a);
-    return hipGetLastError();
+    GridArgs arg = a;
+    void* args[] = {&arg};
+    return hipLaunchKernel(grid_kernel(a.k, a.r), dim3(a.nwg), dim3(64 * a.wg_waves), args, 0, s);
 }
 
 }  // namespace sf

@@ -91,6 +91,7 @@ BatchShape batch_shape(const sf_ctx* c, int nx, int ny);
 BatchShape grid_shape(int nx, int ny);
 struct GridShape {
     int nwg, waves;  // workgroups, waves per workgroup
+    int k, r;        // GridArgs
 };
 GridShape grid_launch_shape(const BatchInstance& d, int k);
 BatchInstance batch_descriptor(const sf_batch_instance& a, int rows, double* q, const double* dt_dev,

@@ -93,6 +93,8 @@ struct PTPlan {
     int r, waves;  // resident: rows per wave, waves
 };
 PTPlan pt_plan(int nx, int ny);
+// The best resident shape with passes launch_us apart, and its modelled time per iteration.
+PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double* us_per_iter);
 hipError_t launch_pt_plan(const PTParams& p, const PTPlan& plan, int k, hipStream_t s);
 // Snapshot staging: dst = (float)(src + shift) (sf_snapshot.hip).
 hipError_t launch_snap_cast(const double* src, float* dst, int64_t n, double shift, hipStream_t s);
@@ -207,7 +209,9 @@ struct BatchResult {
 // arrived, [GRID_SYNC_XCOUNT + 16 x] workgroups on XCD x (one 128-byte line each); part holds
 // 3 * wg_waves * nwg partials.
 enum {
-    GRID_WG_WAVES = 8,
+    GRID_WG_WAVES = 8,         // of the one-wave passes
+    GRID_RESIDENT_WAVES = 16,  // of the resident ones
+    GRID_RESIDENT_MAX_K = 14,
     GRID_MAX_WAVES = 4096,
     GRID_WAIT_SECONDS = 5,
     GRID_MAX_XCD = 16,
@@ -225,15 +229,16 @@ struct GridArgs {
     unsigned long long* sync;
     double* part;
     int nwg, wg_waves;
+    int k, r;        // PT iterations per pass; rows per wave of the resident passes, 0: one-wave passes, k <= 3
     uint64_t limit;  // wall-clock ticks a workgroup may wait at a barrier
 };
 // k = PT iterations per pass (1, 2 or 3; four need more than 256 VGPRs in this kernel); waves =
 // waves per workgroup (1 to GRID_WG_WAVES).
-int grid_capacity(int k, int waves);
+int grid_capacity(int k, int r, int waves);
 uint64_t grid_wait_limit();  // wall-clock ticks of the current limit (sf_set_grid_wait_limit)
 void grid_set_wait_seconds(double seconds);
 double grid_wait_seconds();  // the current limit in seconds
-hipError_t launch_grid_solve(const GridArgs& a, int k, hipStream_t s);
+hipError_t launch_grid_solve(const GridArgs& a, hipStream_t s);
 
 // Wide mode of the batched solver: the active set of one PT-iteration launch.
 #define WIDE_MAX 64

@@ -15,7 +15,7 @@ __global__ __launch_bounds__(64 * PTR_MAX_WAVES) void ptr_tile_f64(PTParams p, i
     __shared__ double lds[PTR_LDS(PTR_MAX_WAVES)];
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int nstrips = p.nstrips;
-    ptr_tile<R>(p, k, logical % nstrips, logical / nstrips, lds);
+    ptr_tile<R>(p, k, p.seg, logical % nstrips, logical / nstrips, lds);
 }
 
 hipError_t launch_pt_resident(const PTParams& p0, int k, int r, int waves, hipStream_t s)
@@ -49,7 +49,7 @@ hipError_t launch_pt_resident(const PTParams& p0, int k, int r, int waves, hipSt
 // Measured against the passes before (us per iteration): 64^2 1.30 (2.6), 301x257 1.64 (3.1), 512^2 2.6
 // (4.65), 700^2 3.85 (about 6.5) resident; 1024^2 6.3 (9.1), 2048^2 19.4 (29.4), 4096^2 69.7 (112)
 // pipelined.  They cross near 730^2: resident 800^2 5.3 against 4.7, pipelined 600^2 3.6 against 2.95.
-PTPlan pt_plan(int nx, int ny)
+PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double* us_per_iter)
 {
     struct Shape {
         int waves, r;
@@ -57,23 +57,32 @@ PTPlan pt_plan(int nx, int ny)
     };
     static const Shape shapes[] = {{8, 1, 0.6, 0.54},  {12, 1, 1.1, 0.61}, {16, 1, 1.6, 0.72}, {8, 2, 1.7, 0.79},
                                    {12, 2, 2.3, 1.01}, {16, 2, 2.9, 1.26}, {12, 3, 3.1, 1.5},  {16, 3, 4.2, 1.85}};
-    static const double step[3] = {0.55, 0.72, 0.94};
     const int cus = 256;
     PTPlan best{};
     double best_us = 1e300;
     if ((int64_t)(nx + 2) * (ny + 2) < PTR_MAX_NODES)
         for (const Shape& sh : shapes)
-            for (int k = 2; k <= PT_PLAN_MAX_K && 2 * k < sh.waves * sh.r; ++k) {
+            for (int k = 2; k <= kmax && 2 * k < sh.waves * sh.r; ++k) {
                 const int out = SF_WAVE - 2 * k, seg = sh.waves * sh.r - 2 * k;
                 const int64_t wgs = (int64_t)((nx - 1 + out - 1) / out) * ((ny + seg - 1) / seg);
                 const double rounds = (double)((wgs + cus - 1) / cus);
                 const double fixed = sh.fixed * (1.0 + 0.5 * std::min(1.0, (double)wgs / cus));
-                const double us = (2.5 + rounds * (fixed + k * sh.iter)) / k;
+                const double us = (launch_us + rounds * (fixed + k * sh.iter)) / k;
                 if (us < best_us) {
                     best_us = us;
                     best = PTPlan{PT_PLAN_RESIDENT, k, 0, sh.r, sh.waves};
                 }
             }
+    *us_per_iter = best_us;
+    return best;
+}
+
+PTPlan pt_plan(int nx, int ny)
+{
+    static const double step[3] = {0.55, 0.72, 0.94};
+    const int cus = 256;
+    double best_us;
+    PTPlan best = pt_plan_resident(nx, ny, PT_PLAN_MAX_K, 2.5, &best_us);
     const int k = PT_PLAN_MAX_K, lag = 9;
     const int strips = (nx - 1 + SF_WAVE - 2 * k - 1) / (SF_WAVE - 2 * k);
     for (int nseg = 1; nseg <= ny && (int64_t)strips * (nseg - 1) < 12 * cus; ++nseg) {

@@ -53,7 +53,7 @@ __device__ __forceinline__ PTRCell ptr_cell(const PTPConst& k, double vx, double
 }
 
 template <int R, class PP>
-__device__ __forceinline__ void ptr_tile(const PP& p, int K, int strip, int segid, double* lds)
+__device__ __forceinline__ void ptr_tile(const PP& p, int K, int seg, int strip, int segid, double* lds)
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -62,7 +62,7 @@ __device__ __forceinline__ void ptr_tile(const PP& p, int K, int strip, int segi
     const int OUT = SF_WAVE - 2 * K;
     const int c0 = strip * OUT - K;
     const int c = c0 + lane;
-    const int r0 = segid * p.seg, r1 = min(r0 + p.seg, ny);
+    const int r0 = segid * seg, r1 = min(r0 + seg, ny);
     const int rw = r0 - K + wave * R;  // the wave's first row
     PTPConst kc;
     kc.rdx = p.rdx;

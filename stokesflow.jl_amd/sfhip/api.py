@@ -283,7 +283,7 @@ def solveStokes_batched(problems, *, mode="auto", rows=0, depth=0, threads=0, ma
     whose working sets fit ``budget_mb`` (default 1536 MiB; 1024 MiB with mixed precision),
     refilled as instances converge; "grid": one instance after another, each solved by one
     launch over the whole chip with the PT loop on the device (``depth`` = PT iterations per
-    pass, 1 to 3, default 3).
+    pass, 1 to 3; default by size).
     ``mixed_precision=True`` (wide mode): every instance is solved as
     ``solveStokes(..., mixed_precision=True)`` solves it (FP32 sweeps inside FP64 defect
     correction), one to three FP32 sweeps per launch of all active instances.
@@ -637,7 +637,7 @@ class StepGraph:
     """The captured timestep of one StokesFlow2D problem (sf_graph_*): the loop body of
     StokesFlow2D_multixpu.jl:164-181 as one hipGraph, the solve with its PT loop on the device
     (one chip-wide launch), RK4 with the new dt read on the device.  Arguments as for
-    :func:`step` (``dt``: the first step's input dt); ``iters_per_pass`` 1 to 3 (0: 3).  The
+    :func:`step` (``dt``: the first step's input dt); ``iters_per_pass`` 1 to 3 (0: by size).  The
     tensors must stay alive while the graph exists.  Bit-identical to repeated :func:`step` calls
     (err to rounding)."""
 
