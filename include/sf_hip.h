@@ -225,7 +225,7 @@ int sf_solve_stokes_refined(sf_ctx *ctx, double *P, double *Vx_pad, double *Vy_p
  * PERSISTENT: one launch; each workgroup takes an instance from a device work queue (largest
  * first), runs its whole solve with the reference's ncheck/ndtupdate rules, exits it on its
  * own convergence, and takes the next (no host synchronisation; capturable).
- * WIDE: one launch per PT iteration covers every instance of an active set whose working
+ * WIDE: a launch of several PT iterations covers every instance of an active set whose working
  * sets fit budget_mb; each instance is checked at its own ncheck iterations and retired on
  * convergence, and the set is refilled from the largest-first queue.
  * GRID: the instances one after another, each solved by ONE launch that spans the chip (at most

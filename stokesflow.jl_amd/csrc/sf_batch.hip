@@ -236,16 +236,9 @@ __global__ __launch_bounds__(BATCH_MAX_THREADS) void batch_solve_kernel(const Ba
 template <int DEPTH>
 __global__ __launch_bounds__(64) void wide_pt_kernel(WideArgs a)
 {
-    const int total = a.tile_start[a.n_active];
-    const int t_glob = xcd_remap(blockIdx.x, gridDim.x);
-    if (t_glob >= total) return;
-    int lo = 0, hi = a.n_active - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.tile_start[mid] <= t_glob) lo = mid;
-        else hi = mid - 1;
-    }
-    const int t = t_glob - a.tile_start[lo];
+    int t;
+    const int lo = wide_slot(a, &t);
+    if (lo < 0) return;
     CBatch* cinst = (CBatch*)a.desc;
     const int pf = a.slot_pf[lo];
     const PTParams SF_CONST& pp = cinst[a.slot_inst[lo]].wpt[pf & 1];
@@ -258,16 +251,9 @@ __global__ __launch_bounds__(64) void wide_pt_kernel(WideArgs a)
 // Two PT iterations of every active instance per launch (pt2_tile, sf_pt2_tile.h).
 __global__ __launch_bounds__(64) void wide_pt2_kernel(WideArgs a)
 {
-    const int total = a.tile_start[a.n_active];
-    const int t_glob = xcd_remap(blockIdx.x, gridDim.x);
-    if (t_glob >= total) return;
-    int lo = 0, hi = a.n_active - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.tile_start[mid] <= t_glob) lo = mid;
-        else hi = mid - 1;
-    }
-    const int t = t_glob - a.tile_start[lo];
+    int t;
+    const int lo = wide_slot(a, &t);
+    if (lo < 0) return;
     CBatch* cinst = (CBatch*)a.desc;
     const PTParams SF_CONST& pp = cinst[a.slot_inst[lo]].wpt[2 + (a.slot_pf[lo] & 1)];
     const int nstrips = pp.nstrips;
@@ -289,16 +275,9 @@ hipError_t launch_wide_pt(const WideArgs& a, int depth, hipStream_t s)
 template <int K, int SPLIT>
 __global__ __launch_bounds__(64) void wide_ptk_kernel(WideArgs a)
 {
-    const int total = a.tile_start[a.n_active];
-    const int t_glob = xcd_remap(blockIdx.x, gridDim.x);
-    if (t_glob >= total) return;
-    int lo = 0, hi = a.n_active - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.tile_start[mid] <= t_glob) lo = mid;
-        else hi = mid - 1;
-    }
-    const int t = t_glob - a.tile_start[lo];
+    int t;
+    const int lo = wide_slot(a, &t);
+    if (lo < 0) return;
     CBatch* cinst = (CBatch*)a.desc;
     const PTParams SF_CONST& pp = cinst[a.slot_inst[lo]].wpt[2 * K - 2 + (a.slot_pf[lo] & 1)];
     const int nstrips = pp.nstrips;

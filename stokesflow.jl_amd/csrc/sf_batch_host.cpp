@@ -117,28 +117,17 @@ BatchInstance batch_descriptor(const sf_batch_instance& a, int rows, double* q, 
         w.dvx_o = par ? a.dVxdtau : dvx2;
         w.dvy_o = par ? a.dVydtau : dvy2;
         b.wpt[par] = w;
-        // at least 4 rows: the wide mode fills the chip with many instances, so the short tiles
-        // that suit one small grid alone would only add halo rows
-        const int rows2 = sh.rows2 > 0 ? std::min(sh.rows2, ny) : std::max(pt2_default_rows(nx, ny), std::min(4, ny));
+        const int rows2 = std::min(ny, sh.rows2 > 0 ? sh.rows2 : pt2_default_rows(nx, ny));
         w.seg = rows2;
         w.nstrips = (nx - 1 + 59) / 60;
         w.ntiles = w.nstrips * ((ny + rows2 - 1) / rows2);
         b.wpt[2 + par] = w;
-        // few instances fill the chip only with shorter tiles: below WIDE_MAX instances the height
-        // comes from the wave-round model over that many copies of the grid (16 x 256^2, one box:
-        // 48-row four-iteration tiles ran 480 waves per launch)
-        const bool model = sh.copies > 0 && sh.copies < WIDE_MAX;
-        const int rows3 = std::min(ny, sh.rows3 > 0 ? sh.rows3
-                                                    : (model ? ptk_default_rows(3, nx, ny, sh.copies)
-                                                             : (std::max(nx, ny) > 256 ? 16 : 8)));
+        const int rows3 = std::min(ny, sh.rows3 > 0 ? sh.rows3 : ptk_default_rows(3, nx, ny));
         w.seg = rows3;
         w.nstrips = (nx - 1 + 57) / 58;
         w.ntiles = w.nstrips * ((ny + rows3 - 1) / rows3);
         b.wpt[4 + par] = w;
-        const int n = std::max(nx, ny);
-        const int rows4 = std::min(ny, sh.rows4 > 0 ? sh.rows4
-                                                    : (model ? ptk_default_rows(4, nx, ny, sh.copies)
-                                                             : (n > 384 ? 64 : (n > 192 ? 48 : 8))));
+        const int rows4 = std::min(ny, sh.rows4 > 0 ? sh.rows4 : ptk_default_rows(4, nx, ny));
         w.seg = rows4;
         w.nstrips = (nx - 1 + 55) / 56;
         w.ntiles = w.nstrips * ((ny + rows4 - 1) / rows4);
@@ -155,11 +144,9 @@ BatchInstance batch_descriptor(const sf_batch_instance& a, int rows, double* q, 
     b.nx = nx;
     b.ny = ny;
     b.use_fss = a.use_fss;
-    // size default: four iterations per pass above 192 nodes per side, three below (wide passes,
-    // ns per node and iteration on the 256-instance ensemble's active sets, best tile heights,
-    // K = 4 / 3: 512^2 0.00691 / 0.00783; 256^2 0.00833 / 0.00905; 128^2 0.01306 / 0.01219;
-    // 64^2 0.03259 / 0.03056)
-    b.kmax = sh.kmax > 0 ? std::min(sh.kmax, 4) : (std::max(nx, ny) > 192 ? 4 : 3);
+    b.kmax = sh.kmax > 0 ? std::min(sh.kmax, 4) : 4;
+    // wide passes by the active set's plan, but for tuned shapes and sizes past its 32-bit offsets
+    b.resident = sh.kmax <= 0 && (int64_t)(nx + 2) * (ny + 2) < PTR_MAX_NODES;
     b.dx = a.dx;
     b.dy = a.dy;
     b.dt_in = a.dt;
@@ -198,17 +185,6 @@ int batch_threads(const sf_batch_params* prm, int* threads, int* rows, const cha
     *rows = (prm && prm->rows > 0) ? prm->rows : 0;  // 0: per instance, pt_default_rows
     if (*threads % 64 != 0 || *threads > 512) return set_err(SF_ERR_ARG, "%s: threads %d", who, *threads);
     return SF_OK;
-}
-
-// Grid mode: the single solver's tile heights for every pass kind (one instance fills the chip).
-BatchShape grid_shape(int nx, int ny)
-{
-    BatchShape sh;
-    sh.kmax = 3;
-    sh.rows2 = std::min(pt2_default_rows(nx, ny), ny);
-    sh.rows3 = std::min(ptk_default_rows(3, nx, ny), ny);
-    sh.rows4 = std::min(ptk_default_rows(4, nx, ny), ny);
-    return sh;
 }
 
 // Grid mode: the launch of an instance.  k = 0: resident passes up to GRID_RESIDENT_NODES.
@@ -284,7 +260,8 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
         int64_t iter, ncheck, ndtupdate;
         double err, ws;
         bool checking;
-        int k;            // iterations of this step's launch (1 to 4)
+        int k;            // iterations of this step's launch
+        int kmax, rows;   // the plan's
         int64_t nlaunch;  // launches so far: their parity says where the state (V, P, dV) is
         // A check's err is read one step later: the host waits for the step before the one it
         // has just enqueued, so the GPU never drains at a check.  Meanwhile the instance may run
@@ -302,7 +279,7 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
         const sf_batch_instance& a = in[id];
         const int mn = std::min(a.nx, a.ny);
         Run r{id, 1, std::min<int64_t>(5 * (int64_t)mn, 2000), 10 * (int64_t)mn, 2.0 * a.eps,
-              batch_working_set(a.nx, a.ny), false, 1, 0, false, false, 0, 0};
+              batch_working_set(a.nx, a.ny), false, 1, 1, 0, 0, false, false, 0, 0};
         HIPCHK(launch_set_scalar(desc[(size_t)id].scal + SC_DT, a.use_fss ? a.dt : 0.0, s));
         act.push_back(r);
         ws_active += r.ws;
@@ -346,11 +323,17 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
     for (int k = 0; k < 2; ++k) HIPCHK(hipEventCreateWithFlags(&ev.e[k], hipEventDisableTiming));
     bool step_checked[2] = {false, false};
     int64_t step = 0;
-    WideArgs wa, w2, w3, w4;
+    WideArgs wa, w2, w3, w4, wr, wp;
+    WidePlan plan{};      // of the resident passes, for the active instances without a tuned shape
+    bool replan = true;   // the active set has changed
     std::memset(&wa, 0, sizeof(wa));
     std::memset(&w2, 0, sizeof(w2));
     std::memset(&w3, 0, sizeof(w3));
     std::memset(&w4, 0, sizeof(w4));
+    std::memset(&wr, 0, sizeof(wr));
+    std::memset(&wp, 0, sizeof(wp));
+    wr.desc = env.desc_dev;
+    wp.desc = env.desc_dev;
     wa.desc = env.desc_dev;
     w2.desc = env.desc_dev;
     w3.desc = env.desc_dev;
@@ -360,14 +343,33 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
                (act.empty() || ws_active + batch_working_set(in[order[q]].nx, in[order[q]].ny) <= budget)) {
             rc = start(order[q++]);
             if (rc) return rc;
+            replan = true;
         }
-        // every active instance advances by three or two PT iterations in one pass where its next
-        // iterations are plain (the rule of sf_solve_stokes), else by one; each kind is a launch
+        if (replan) {
+            int nx[WIDE_MAX], ny[WIDE_MAX], k[WIDE_MAX], rows[WIDE_MAX], m = 0;
+            for (const Run& r : act)
+                if (desc[(size_t)r.id].resident) {
+                    nx[m] = in[r.id].nx;
+                    ny[m++] = in[r.id].ny;
+                }
+            if (m > 0) plan = wide_plan(nx, ny, m, k, rows);
+            m = 0;
+            for (Run& r : act)
+                if (desc[(size_t)r.id].resident) {
+                    r.kmax = k[m];
+                    r.rows = rows[m++];
+                }
+            replan = false;
+        }
+        // every active instance advances by as many PT iterations in one pass as its plan has and its
+        // next plain iterations allow (the rule of sf_solve_stokes), else by one; each kind is a launch
+        wr.n_active = 0;
+        wp.n_active = 0;
         wa.n_active = 0;
         w2.n_active = 0;
         w3.n_active = 0;
         w4.n_active = 0;
-        int tiles = 0, tiles2 = 0, tiles3 = 0, tiles4 = 0;
+        int tiles = 0, tiles2 = 0, tiles3 = 0, tiles4 = 0, tiles_r = 0, tiles_p = 0;
         for (size_t k = 0; k < act.size(); ++k) {
             Run& r = act[k];
             const sf_batch_instance& a = in[r.id];
@@ -381,9 +383,9 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
                 }
                 return true;
             };
-            const int kmax = desc[(size_t)r.id].kmax;
+            const bool resident = desc[(size_t)r.id].resident;
             r.k = 1;
-            for (int kk = kmax; kk >= 2 && r.k == 1; --kk)
+            for (int kk = resident ? r.kmax : desc[(size_t)r.id].kmax; kk >= 2 && r.k == 1; --kk)
                 if (fusable(kk)) r.k = kk;
             r.checking = check;
             // while its check is pending an instance runs only a plain pass
@@ -391,7 +393,22 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
                                 (a.use_fss && (r.iter + r.k - 1) % r.ndtupdate == 0));
             if (r.skip) continue;
             const int par = (int)(r.nlaunch & 1);
-            if (r.k == 4) {
+            if (resident && plan.pipe && r.k == WIDE_PIPE_K) {
+                wp.tile_start[wp.n_active] = tiles_p;
+                wp.slot_inst[wp.n_active] = r.id;
+                wp.slot_pf[wp.n_active] = par;
+                wp.slot_rows[wp.n_active] = r.rows;
+                tiles_p += wide_pipe_tiles(a.nx, a.ny, r.rows);
+                wp.n_active += 1;
+            } else if (resident && !check && !last) {
+                wr.tile_start[wr.n_active] = tiles_r;
+        wp.tile_start[wp.n_active] = tiles_p;
+        if (wp.n_active) HIPCHK(launch_wide_pipe(wp, s));
+                wr.slot_inst[wr.n_active] = r.id;
+                wr.slot_pf[wr.n_active] = par | (r.k << 1);
+                tiles_r += wide_resident_tiles(plan, a.nx, a.ny, r.k);
+                wr.n_active += 1;
+            } else if (r.k == 4) {
                 w4.tile_start[w4.n_active] = tiles4;
                 w4.slot_inst[w4.n_active] = r.id;
                 w4.slot_pf[w4.n_active] = par;
@@ -422,6 +439,10 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
         w2.tile_start[w2.n_active] = tiles2;
         w3.tile_start[w3.n_active] = tiles3;
         w4.tile_start[w4.n_active] = tiles4;
+        wr.tile_start[wr.n_active] = tiles_r;
+        wp.tile_start[wp.n_active] = tiles_p;
+        if (wp.n_active) HIPCHK(launch_wide_pipe(wp, s));
+        if (wr.n_active) HIPCHK(launch_wide_resident(wr, plan, s));
         if (w4.n_active) HIPCHK(launch_wide_pt4(w4, s));
         if (w3.n_active) HIPCHK(launch_wide_pt3(w3, s));
         if (w2.n_active) HIPCHK(launch_wide_pt2(w2, s));
@@ -523,6 +544,7 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
                 ws_active -= r.ws;
             }
         }
+        replan = keep.size() != act.size();
         act.swap(keep);
         ++step;
     }
@@ -1013,8 +1035,7 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
     const int precision = prm ? prm->precision : 0;
     std::vector<BatchInstance> host((size_t)n);
     for (int i = 0; i < n; ++i) {
-        BatchShape sh = mode == SF_BATCH_GRID ? grid_shape(in[i].nx, in[i].ny) : batch_shape(c, in[i].nx, in[i].ny);
-        if (mode != SF_BATCH_GRID) sh.copies = n;
+        const BatchShape sh = mode == SF_BATCH_GRID ? BatchShape() : batch_shape(c, in[i].nx, in[i].ny);
         host[(size_t)i] = batch_descriptor(in[i], rows, c->b_pool + off[(size_t)i], nullptr, sh);
     }
     std::vector<std::pair<int, int>> dims((size_t)n);

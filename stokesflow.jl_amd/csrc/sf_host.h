@@ -74,21 +74,17 @@ struct RefineEnv {
 size_t batch_scratch_doubles(int nx, int ny);
 int batch_check(const sf_batch_instance& a, int i, const char* who);
 
-// Launch shape of an instance's wide FP64 passes (results do not depend on it): the most PT
-// iterations per pass (2, 3 or 4) and the tile rows of the two-, three- and four-iteration
+// Tuned launch shape of an instance's wide FP64 passes (results do not depend on it): the most PT
+// iterations per pass (2, 3 or 4; 0: not tuned, wide_plan's passes) and the tile rows of the two-, three- and four-iteration
 // passes (0: size default).  sf_batch_autotune keeps one per grid size on the context.
 struct BatchShape {
     int kmax = 0, rows2 = 0, rows3 = 0, rows4 = 0;
-    // instances of the batch: below WIDE_MAX the default three- and four-iteration tile heights
-    // come from the wave-round model over that many copies of the grid (0: the fixed table)
-    int copies = 0;
 };
 struct BatchTune {
     int nx, ny;
     BatchShape sh;
 };
 BatchShape batch_shape(const sf_ctx* c, int nx, int ny);
-BatchShape grid_shape(int nx, int ny);
 struct GridShape {
     int nwg, waves;  // workgroups, waves per workgroup
     int k, r;        // GridArgs

@@ -77,7 +77,7 @@ int pt2_default_rows(int nx, int ny);
 // p.seg <= 0: ptk_default_rows).
 hipError_t launch_pt_multi(const PTParams& p, int k, hipStream_t s);
 // tile height of a k-iteration pass (k >= 3) when `copies` grids of this size share the launch
-int ptk_default_rows(int k, int nx, int ny, int copies = 1);
+int ptk_default_rows(int k, int nx, int ny);
 // k = 5, 6 or 7 PT iterations per pass, pipelined over the waves of a workgroup (sf_ptp_tile.h), in
 // tiles of `rows` rows.
 hipError_t launch_pt_pipe(const PTParams& p, int k, int rows, hipStream_t s);
@@ -189,7 +189,8 @@ struct BatchInstance {
     double *P, *Vx_s, *Vy_s, *Vx_pad, *Vy_pad;  // caller state (in/out)
     double *ry, *scal;                          // library scratch (scal[SC_DT] = stabilisation dt)
     const double* dt_dev;                       // if set, the input dt is read here (device) instead of dt_in
-    int nx, ny, use_fss, kmax;  // kmax: most PT iterations per wide pass (2, 3 or 4)
+    int nx, ny, use_fss, kmax;  // kmax: most PT iterations per one-wave wide pass (2, 3 or 4)
+    int resident, pad;          // wide passes on tiles in registers (no tuned shape)
     double dx, dy, dt_in, maxdisp, eps;
     int64_t iter_max;
 };
@@ -247,7 +248,8 @@ struct WideArgs {
     int n_active;
     int tile_start[WIDE_MAX + 1];  // prefix of the slots' tile counts
     int slot_inst[WIDE_MAX];       // descriptor index
-    int slot_pf[WIDE_MAX];         // ping-pong parity | PT_WRITE_* flags << 1
+    int slot_pf[WIDE_MAX];         // ping-pong parity | PT_WRITE_* flags << 1 (resident passes: iterations << 1)
+    int slot_rows[WIDE_MAX];       // pipelined passes: rows per tile
 };
 // One PT iteration of every slot (descriptor wpt[parity]).
 hipError_t launch_wide_pt(const WideArgs& a, int depth, hipStream_t s);
@@ -257,6 +259,22 @@ hipError_t launch_wide_pt2(const WideArgs& a, hipStream_t s);
 hipError_t launch_wide_pt3(const WideArgs& a, hipStream_t s);
 // Four PT iterations of every slot (descriptor wpt[6 + parity]).
 hipError_t launch_wide_pt4(const WideArgs& a, hipStream_t s);
+// Passes on tiles in registers (sf_ptr_tile.h): slot i runs slot_pf[i] >> 1 iterations (parity in bit 0)
+// on descriptor wpt[parity].
+#define WIDE_RESIDENT_MAX_K 14
+// WIDE_PIPE_K iterations of every slot pipelined over waves (sf_ptp_tile.h) in tiles of slot_rows[i] rows.
+#define WIDE_PIPE_K 7
+hipError_t launch_wide_pipe(const WideArgs& a, hipStream_t s);
+int wide_pipe_tiles(int nx, int ny, int rows);
+// The plan holds for one set of grids: k[i] = the most iterations per pass, rows[i] = the tile height of
+// the pipelined passes.
+struct WidePlan {
+    int pipe;      // passes of WIDE_PIPE_K iterations are pipelined, shorter ones resident
+    int r, waves;  // resident shape
+};
+WidePlan wide_plan(const int* nx, const int* ny, int n, int* k, int* rows);
+int wide_resident_tiles(const WidePlan& plan, int nx, int ny, int k);
+hipError_t launch_wide_resident(const WideArgs& a, const WidePlan& plan, hipStream_t s);
 
 // Wide mode of the FP32 correction sweeps: slot k runs descriptor slot_desc[k] (two
 // descriptors per instance, one per ping-pong direction).

@@ -24,6 +24,24 @@ __device__ inline int xcd_remap(int k, int total)
     return (xcd < rem) ? xcd * (bpx + 1) + idx : rem * (bpx + 1) + (xcd - rem) * bpx + idx;
 }
 
+typedef const BatchInstance __attribute__((address_space(4))) WideInstC;
+
+// Wide launches: the slot whose tiles this workgroup's lies among, and the tile *t within it; -1 past
+// the last.  The tile order is XCD-banded, so an XCD works on consecutive grids.
+__device__ inline int wide_slot(const WideArgs& a, int* t)
+{
+    const int t_glob = xcd_remap(blockIdx.x, gridDim.x);
+    if (t_glob >= a.tile_start[a.n_active]) return -1;
+    int lo = 0, hi = a.n_active - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.tile_start[mid] <= t_glob) lo = mid;
+        else hi = mid - 1;
+    }
+    *t = t_glob - a.tile_start[lo];
+    return lo;
+}
+
 
 // Operands one row step consumes (row r of the cell/basic quantities, row r+1 of V/rho,
 // row r-1 of dVx/dVy).

@@ -11,7 +11,7 @@ __global__ __launch_bounds__(64 * PTPShape<K>::WAVES, 3) void ptp_tile_f64(PTPar
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int nstrips = p.nstrips;
     // the kernel's only argument, read in place
-    ptp_tile<K>(*(PTParamsC*)__builtin_amdgcn_kernarg_segment_ptr(), logical % nstrips, logical / nstrips, lds);
+    ptp_tile<K>(*(PTParamsC*)__builtin_amdgcn_kernarg_segment_ptr(), p.seg, logical % nstrips, logical / nstrips, lds);
 }
 
 template <int K>
@@ -34,6 +34,34 @@ hipError_t launch_pt_pipe(const PTParams& p, int k, int rows, hipStream_t s)
         case 7: return launch_k<7>(p, rows, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+// The tiles of several grids (the wide batched mode): slot i in tiles of slot_rows[i] rows.
+template <int K>
+__global__ __launch_bounds__(64 * PTPShape<K>::WAVES, 3) void wide_ptp_kernel(WideArgs a)
+{
+    __shared__ double lds[PTPShape<K>::LDS];
+    int t;
+    const int i = wide_slot(a, &t);
+    if (i < 0) return;
+    PTParamsC& pp = ((WideInstC*)a.desc)[a.slot_inst[i]].wpt[a.slot_pf[i] & 1];
+    const int nstrips = (pp.nx - 1 + PTPShape<K>::OUT - 1) / PTPShape<K>::OUT;
+    ptp_tile<K>(pp, a.slot_rows[i], t % nstrips, t / nstrips, lds);
+}
+
+int wide_pipe_tiles(int nx, int ny, int rows)
+{
+    return ((nx - 1 + PTPShape<WIDE_PIPE_K>::OUT - 1) / PTPShape<WIDE_PIPE_K>::OUT) * ((ny + rows - 1) / rows);
+}
+
+hipError_t launch_wide_pipe(const WideArgs& a, hipStream_t s)
+{
+    const int total = a.tile_start[a.n_active];
+    if (total <= 0) return hipSuccess;
+    for (int i = 0; i < a.n_active; ++i)
+        if (a.slot_rows[i] < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(wide_ptp_kernel<WIDE_PIPE_K>, dim3(total), dim3(64 * PTPShape<WIDE_PIPE_K>::WAVES), 0, s, a);
+    return hipGetLastError();
 }
 
 }  // namespace sf

@@ -485,11 +485,11 @@ __device__ __forceinline__ PTParamsC& ptp_fresh(PTParamsC& p)
     return *q;
 }
 
-// K PT iterations over the tile (strip, segid) by the PTPShape<K>::WAVES waves of a workgroup:
+// K PT iterations over the tile (strip, segid) of seg rows by the PTPShape<K>::WAVES waves of a workgroup:
 // state k from (vx_a, vy_a, p_a, dvx, dvy), state k+K to (vx_b, vy_b, p_b, dvx_o, dvy_o); lds holds
 // PTPShape<K>::LDS doubles.  Every wave of the workgroup calls this (one barrier per step).
 template <int K>
-__device__ __forceinline__ void ptp_tile(PTParamsC& p, int strip, int segid, double* lds)
+__device__ __forceinline__ void ptp_tile(PTParamsC& p, int seg, int strip, int segid, double* lds)
 {
     typedef PTPShape<K> S;
     const int lane = threadIdx.x & 63;
@@ -497,8 +497,8 @@ __device__ __forceinline__ void ptp_tile(PTParamsC& p, int strip, int segid, dou
     const int nx = p.nx, ny = p.ny;
     const int c0 = strip * S::OUT - (K - 1);
     const int c = c0 + lane;
-    const int r0 = segid * p.seg;
-    const int r1 = min(r0 + p.seg, ny);
+    const int r0 = segid * seg;
+    const int r1 = min(r0 + seg, ny);
     const int rstart = max(r0 - K, 0);
     const int steps = r1 - rstart + S::LAG;
     PTPEdge e;

@@ -279,7 +279,7 @@ def solveStokes_batched(problems, *, mode="auto", rows=0, depth=0, threads=0, ma
     runtime = wall time of the whole batch).
 
     ``mode`` "persistent": one launch, one workgroup per instance from a device work queue;
-    "wide" (= "auto"): one to four PT iterations per launch over an active set of instances
+    "wide" (= "auto"): up to 14 PT iterations per launch over an active set of instances
     whose working sets fit ``budget_mb`` (default 1536 MiB; 1024 MiB with mixed precision),
     refilled as instances converge; "grid": one instance after another, each solved by one
     launch over the whole chip with the PT loop on the device (``depth`` = PT iterations per

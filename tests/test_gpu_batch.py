@@ -270,3 +270,22 @@ def test_batch_autotune_keeps_results(gpu):
         assert o["niter"] == st["niter"] and o["dt_new"] == st["dt_new"], (nx, ny)
         for k in OUT:
             assert np.array_equal(sfhip.to_numpy(G[k]), exp[k]), (nx, ny, k)
+
+
+@pytest.mark.parametrize("sizes,cap", [
+    ([(64, 64)], 643),                                          # one small grid
+    ([(33, 47), (200, 90), (17, 90), (64, 200)], 211),          # tiles for a part of the chip
+    ([(256, 200), (131, 300), (256, 257)] * 6, 700),            # pipelined passes, short ones before checks
+    ([(3, 3), (3, 64), (64, 3), (600, 520), (500, 640)], 60),   # uneven sizes in one launch
+])
+def test_wide_default_passes(gpu, sizes, cap):
+    insts = [(nx, ny, cases.smooth_state(nx, ny, seed=40 + k)) for k, (nx, ny) in enumerate(sizes)]
+    probs = [problem(S, nx, ny, 1.0 / (nx - 1), 1.0 / (ny - 1), iterMax=cap) for nx, ny, S in insts]
+    outs = sfhip.solveStokes_batched([p for p, _ in probs], mode="wide")
+    torch.cuda.synchronize()
+    for (nx, ny, S), (_, G), o in zip(insts, probs, outs):
+        st, exp = single(S, nx, ny, 1.0 / (nx - 1), 1.0 / (ny - 1), iterMax=cap)
+        assert o["niter"] == st["niter"] and o["dt_new"] == st["dt_new"], (nx, ny)
+        assert o["err"] == pytest.approx(st["err"], rel=1e-12, abs=0.0)
+        for k in OUT:
+            assert np.array_equal(sfhip.to_numpy(G[k]), exp[k]), (nx, ny, k)
