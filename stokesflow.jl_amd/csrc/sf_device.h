@@ -74,4 +74,19 @@ __device__ __forceinline__ T lane_up(T v, int d)
     return v;
 }
 
+// a / b without range scaling and special cases: the steps of the IEEE division sequence (the
+// reciprocal refined twice, one remainder step), hence its bits, where every operand and quotient lies
+// far inside the normal range.  A divisor's reciprocal y is formed once for a constant.
+__device__ __forceinline__ double ptp_div_by(double a, double b, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+__device__ __forceinline__ double ptp_recip(double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    return __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+}
+
 }  // namespace sf

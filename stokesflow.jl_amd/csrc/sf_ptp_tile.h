@@ -131,20 +131,6 @@ __device__ __forceinline__ void ptp_bc(const PTPEdge& e, bool last_row, double& 
     if (last_row) vy = 0.0;
 }
 
-// a / b without range scaling and special cases: the steps of the IEEE division sequence (the
-// reciprocal refined twice, one remainder step), hence its bits, where every operand and quotient lies
-// far inside the normal range.  A divisor's reciprocal y is formed once for a constant.
-__device__ __forceinline__ double ptp_div_by(double a, double b, double y)
-{
-    const double q = a * y;
-    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
-}
-__device__ __forceinline__ double ptp_recip(double b)
-{
-    double y = __builtin_amdgcn_rcp(b);
-    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
-    return __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
-}
 // Whether the divisions of the pseudo-time steps stay in that range: mu_p of the row and the
 // constants within 2^+-200 on every lane (a uniform test; else the divisions are full ones).  Wave 0
 // issues 131 instead of 162 VALU instructions per row: 79.2 -> 71.2 us per iteration at 4096^2 together

@@ -4,7 +4,11 @@
 // (:181-187): one thread per marker, four stages of two bilinear gathers plus the
 // continuity-based second-order correction, the failsafe index clamps, and the final
 // clamp to [0, lx] x [0, ly].  Same IEEE operations in the same order as the reference,
-// so positions are bit-identical to a CPU evaluation.  Marker arrays keep their order.
+// so positions are bit-identical to a CPU evaluation.  Marker arrays keep their order.  Waves of ordinary
+// markers take interp_plain, which has the same bits; interp_v serves every input.
+#include <algorithm>
+#include <cmath>
+
 #include "sf_device.h"
 #include "sf_internal.h"
 
@@ -85,12 +89,91 @@ __device__ inline bool interp_v(double x, double y, const double* __restrict__ V
     return true;
 }
 
+// Whether interp_plain may take a launch (by the host), and how far from the origin a marker may be.
+struct RKPlain {
+    bool ok;
+    double xlim, ylim;
+};
+
+typedef double rk_pair __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte loads need no more alignment
+
+// The velocities around a marker, kept from stage to stage.
+struct RKCell {
+    unsigned ox, oy;  // byte offsets of a and c in Vx and Vy
+    rk_pair a01, b01, c0, c1, c2;
+    double a2, b2;
+};
+
+// interp_v for plain markers (see rk4_kernel): the same bits with half the instructions.  Divisions
+// by dx and dy are three steps with one reciprocal each; floor gives the index without 64-bit
+// conversions; the three neighbours of the correction lie in a row that starts at the cell's node or
+// one before it, so both cases read three consecutive values; clamps are tested once for the wave.
+// Most markers stay in their half cell from stage to stage, and only the others load again (fewer
+// than half the cache accesses: lanes lie rows apart, so nearly every lane is an access of its own).
+// 268 M markers on 4096^2 nodes take 5.6 ms, 10.3 by interp_v alone; VALU issue bounds it (654
+// instructions per wave, 91% of the cycles), two thirds of them the FP64 operations of the formulas.
+__device__ inline void interp_plain(double x, double y, bool first, RKCell& q, const double* __restrict__ Vx, int n1x,
+                                    int n2x, const double* __restrict__ Vy, int n1y, int n2y, double x_vx_min,
+                                    double y_vx_min, double x_vy_min, double y_vy_min, double dx, double dy, double rdx,
+                                    double rdy, double& vx, double& vy, int& nclamp)
+{
+    double fx = floor(ptp_div_by(x - x_vx_min, dx, rdx)), fy = floor(ptp_div_by(y - y_vx_min, dy, rdy));
+    double dxij = ptp_div_by(x - (x_vx_min + fx * dx), dx, rdx), dyij = ptp_div_by(y - (y_vx_min + fy * dy), dy, rdy);
+    int i = (int)fx, j = (int)fy;  // 0-based
+    fx = floor(ptp_div_by(x - x_vy_min, dx, rdx));
+    fy = floor(ptp_div_by(y - y_vy_min, dy, rdy));
+    double exij = ptp_div_by(x - (x_vy_min + fx * dx), dx, rdx), eyij = ptp_div_by(y - (y_vy_min + fy * dy), dy, rdy);
+    int k = (int)fx, l = (int)fy;
+    const bool inside = (unsigned)(i - 1) < (unsigned)(n1x - 3) && (unsigned)j < (unsigned)(n2x - 1) &&
+                        (unsigned)k < (unsigned)(n1y - 1) && (unsigned)(l - 1) < (unsigned)(n2y - 3);
+    if (__ballot(!inside)) {
+        if (i < 1) { i = 1; dxij = 0.0; ++nclamp; }
+        if (j < 0) { j = 0; dyij = 0.0; ++nclamp; }
+        if (i >= n1x - 2) { i = n1x - 3; dxij = 1.0; ++nclamp; }
+        if (j >= n2x - 1) { j = n2x - 2; dyij = 1.0; ++nclamp; }
+        if (k < 0) { k = 0; exij = 0.0; ++nclamp; }
+        if (l < 1) { l = 1; eyij = 0.0; ++nclamp; }
+        if (k >= n1y - 1) { k = n1y - 2; exij = 1.0; ++nclamp; }
+        if (l >= n2y - 2) { l = n2y - 3; eyij = 1.0; ++nclamp; }
+    }
+    const bool right = dxij >= 0.5, down = eyij >= 0.5;
+    const unsigned ox = 8u * (__umul24(j, n1x) + (unsigned)(right ? i : i - 1));
+    const unsigned oy = 8u * (__umul24(down ? l : l - 1, n1y) + (unsigned)k);
+    if (first || ox != q.ox) {
+        const char *a = (const char*)Vx, *b = (const char*)(Vx + n1x);
+        q.a01 = *(const rk_pair*)(a + ox);
+        q.a2 = *(const double*)(a + ox + 16);
+        q.b01 = *(const rk_pair*)(b + ox);
+        q.b2 = *(const double*)(b + ox + 16);
+        q.ox = ox;
+    }
+    if (first || oy != q.oy) {
+        q.c0 = *(const rk_pair*)((const char*)Vy + oy);
+        q.c1 = *(const rk_pair*)((const char*)(Vy + n1y) + oy);
+        q.c2 = *(const rk_pair*)((const char*)(Vy + n1y + n1y) + oy);
+        q.oy = oy;
+    }
+    const double hx = dxij - 0.5, hy = eyij - 0.5;
+    vx = bilinear(right ? q.a01.x : q.a01.y, right ? q.a01.y : q.a2, right ? q.b01.x : q.b01.y, right ? q.b01.y : q.b2,
+                  dxij, dyij) +
+         (0.5 * (hx * hx)) *
+             ((1.0 - dyij) * ((q.a01.x - 2.0 * q.a01.y) + q.a2) + dyij * ((q.b01.x - 2.0 * q.b01.y) + q.b2));
+    vy = bilinear(down ? q.c0.x : q.c1.x, down ? q.c0.y : q.c1.y, down ? q.c1.x : q.c2.x, down ? q.c1.y : q.c2.y, exij,
+                  eyij) +
+         (0.5 * (hy * hy)) *
+             ((1.0 - exij) * ((q.c0.x - 2.0 * q.c1.x) + q.c2.x) + exij * ((q.c0.y - 2.0 * q.c1.y) + q.c2.y));
+}
+
+// A wave whose markers are all plain takes interp_plain.  Plain: starting 2^-200 or more from the axes,
+// and in every stage at most 2^28 cells from the origin.  Then no stage's position is -0 or has bits
+// below 2^-320, and with grid lines and spacings as the host requires every difference to a grid line
+// is +0 or at least 2^-380: no operand, quotient or remainder of a division leaves the normal range.
 __global__ __launch_bounds__(256) void rk4_kernel(double* __restrict__ x_m, double* __restrict__ y_m, int64_t nm,
                                                   const double* __restrict__ Vx, int n1x, int n2x,
                                                   const double* __restrict__ Vy, int n1y, int n2y, double x_vx_min,
                                                   double y_vx_min, double x_vy_min, double y_vy_min, double dt_val,
                                                   const double* __restrict__ dt_ptr, double lx, double ly, double dx,
-                                                  double dy, unsigned long long* __restrict__ counters)
+                                                  double dy, RKPlain plain, unsigned long long* __restrict__ counters)
 {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= nm) return;
@@ -100,16 +183,36 @@ __global__ __launch_bounds__(256) void rk4_kernel(double* __restrict__ x_m, doub
     const double x_old = x_m[m], y_old = y_m[m];
     double vx_eff = 0.0, vy_eff = 0.0, vx_rk = 0.0, vy_rk = 0.0;
     int nclamp = 0;
-    for (int it = 0; it < 4; ++it) {
-        const double x_rk = x_old + rk_dt[it] * vx_rk;
-        const double y_rk = y_old + rk_dt[it] * vy_rk;
-        if (!interp_v(x_rk, y_rk, Vx, n1x, n2x, Vy, n1y, n2y, x_vx_min, y_vx_min, x_vy_min, y_vy_min, dx, dy, vx_rk,
-                      vy_rk, nclamp)) {
-            atomicAdd(&counters[RK_NONFINITE], 1ull);
-            return;
+    bool done = plain.ok && !__ballot(!(fabs(x_old) >= 0x1p-200 && fabs(y_old) >= 0x1p-200));
+    if (done) {
+        const double rdx = ptp_recip(dx), rdy = ptp_recip(dy);
+        RKCell cell;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const double x_rk = it ? x_old + rk_dt[it] * vx_rk : x_old;
+            const double y_rk = it ? y_old + rk_dt[it] * vy_rk : y_old;
+            done = !__ballot(!(fabs(x_rk) <= plain.xlim && fabs(y_rk) <= plain.ylim));
+            if (!done) break;
+            interp_plain(x_rk, y_rk, it == 0, cell, Vx, n1x, n2x, Vy, n1y, n2y, x_vx_min, y_vx_min, x_vy_min, y_vy_min, dx,
+                         dy, rdx, rdy, vx_rk, vy_rk, nclamp);
+            vx_eff = vx_eff + rk_wt[it] * vx_rk;
+            vy_eff = vy_eff + rk_wt[it] * vy_rk;
         }
-        vx_eff = vx_eff + rk_wt[it] * vx_rk;
-        vy_eff = vy_eff + rk_wt[it] * vy_rk;
+    }
+    if (!done) {
+        vx_eff = vy_eff = vx_rk = vy_rk = 0.0;
+        nclamp = 0;
+        for (int it = 0; it < 4; ++it) {
+            const double x_rk = x_old + rk_dt[it] * vx_rk;
+            const double y_rk = y_old + rk_dt[it] * vy_rk;
+            if (!interp_v(x_rk, y_rk, Vx, n1x, n2x, Vy, n1y, n2y, x_vx_min, y_vx_min, x_vy_min, y_vy_min, dx, dy, vx_rk,
+                          vy_rk, nclamp)) {
+                atomicAdd(&counters[RK_NONFINITE], 1ull);
+                return;
+            }
+            vx_eff = vx_eff + rk_wt[it] * vx_rk;
+            vy_eff = vy_eff + rk_wt[it] * vy_rk;
+        }
     }
     const double x_new = x_old + vx_eff * dt;
     const double y_new = y_old + vy_eff * dt;
@@ -278,8 +381,15 @@ hipError_t launch_rk4(double* x_m, double* y_m, int64_t nm, const double* vx, in
                       const double* dt_ptr)
 {
     if (nm <= 0) return hipSuccess;
+    auto spacing = [](double d) { return d > 0x1p-200 && d < 0x1p200; };
+    auto origin = [](double c, double d) { return c == 0.0 || (fabs(c) >= 0x1p-300 && fabs(c) <= 0x1p28 * d); };
+    const bool small = 8.0 * vx_n1 * vx_n2 < 0x1p32 && 8.0 * vy_n1 * vy_n2 < 0x1p32 &&  // 32-bit byte offsets
+                       std::max(std::max(vx_n1, vx_n2), std::max(vy_n1, vy_n2)) < 1 << 24;
+    const RKPlain plain{small && spacing(dx) && spacing(dy) && origin(x_vx_min, dx) && origin(y_vx_min, dy) &&
+                            origin(x_vy_min, dx) && origin(y_vy_min, dy),
+                        0x1p28 * dx, 0x1p28 * dy};
     hipLaunchKernelGGL(rk4_kernel, dim3(g1(nm)), dim3(256), 0, s, x_m, y_m, nm, vx, vx_n1, vx_n2, vy, vy_n1, vy_n2,
-                       x_vx_min, y_vx_min, x_vy_min, y_vy_min, dt, dt_ptr, lx, ly, dx, dy, counters);
+                       x_vx_min, y_vx_min, x_vy_min, y_vy_min, dt, dt_ptr, lx, ly, dx, dy, plain, counters);
     return hipGetLastError();
 }
 

@@ -158,6 +158,25 @@ def test_rk4_bitwise_vs_oracle(gpu, nx, ny, seed):
     assert st["n_clamped"] == nc and nc > 0
 
 
+@pytest.mark.parametrize("nx,ny,n", [(3, 3, 700), (40, 29, 703), (130, 67, 1)])
+def test_rk4_plain_and_general_waves_vs_oracle(gpu, nx, ny, n):
+    """Waves of ordinary markers beside waves with one on an axis, next to one, outside, or far away."""
+    rng = np.random.default_rng(nx + n)
+    dx, dy = 1.0 / (nx - 1), 0.7 / (ny - 1)
+    Vx = np.asfortranarray(rng.random((nx + 2, ny + 1)) - 0.5)
+    Vy = np.asfortranarray(rng.random((nx + 1, ny + 2)) - 0.5)
+    x, y = rng.random(n), 0.7 * rng.random(n)
+    if n > 650:
+        x[70], y[140], x[200], y[270], x[330] = 0.0, -0.0, 1e-310, -1e-250, -2.5
+        y[400], x[460], y[530], x[600] = 40.0, 1e9 * dx, -1e12 * dy, 1e-130
+    dt = 2.0 * min(dx / np.max(np.abs(Vx)), dy / np.max(np.abs(Vy)))  # several cells: the stages lie apart
+    gx, gy, st = rk4_gpu(x, y, Vx, Vy, dx, dy, dt, 1.0, 0.7)
+    ex, ey = x.copy(), y.copy()
+    nc = O.move_markers_rk4(ex, ey, Vx, Vy, -dx, -0.5 * dy, -0.5 * dx, -dy, dt, 1.0, 0.7, dx, dy)
+    assert gx.tobytes() == ex.tobytes() and gy.tobytes() == ey.tobytes()
+    assert st["n_clamped"] == nc
+
+
 def test_rk4_constant_velocity(gpu, golden):
     c = golden["move_markers_constant"]
     nx, ny, dx, dy = c["nx"], c["ny"], c["dx"], c["dy"]
