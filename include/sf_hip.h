@@ -82,11 +82,13 @@ int sf_ctx_set_pt_tuning(sf_ctx *ctx, int rows, int depth, int max_waves);
 /* Temporal blocking of the PT iteration: iters_per_launch = 2, 3 or 4 runs that many plain
  * iterations (no check iteration, no dt refresh before the last of them, not the last
  * iteration or the first timed one) as one pass that reads and writes the state once (where
- * they do not fit, shorter passes); 1 runs one iteration per launch; 0 is the size default (4
- * above 448 nodes per side, else 2).  The FP32 sweeps of sf_solve_stokes_refined take the same
- * setting with 5 also allowed (the FP64 passes cap it at 4); their default is 5 above 3072
- * nodes per side, 4 above 1536, 3 above 768, else 2.
- * rows: grid rows per tile of the pass (0 = size default).  Results are bit-identical either
+ * they do not fit, shorter passes); 1 runs one iteration per launch; 0 is the size default
+ * (passes of up to 7 iterations held in registers or pipelined over a workgroup's waves).  The
+ * FP32 sweeps of sf_solve_stokes_refined take the same setting with 5 also allowed (the FP64
+ * passes cap it at 4); their default is 5 above 3072 nodes per side, else up to 12 by size, held
+ * in registers.
+ * rows: grid rows per tile of the pass (0 = size default; with rows alone, one-wave passes of a
+ * default length).  Results are bit-identical either
  * way; the pass needs a second dVx/dVy buffer, allocated in the context on first use.  No
  * reference counterpart (the reference launches each of its kernels once per iteration). */
 int sf_ctx_set_pt_fusion(sf_ctx *ctx, int iters_per_launch, int rows);

@@ -593,16 +593,12 @@ RefineBufs refine_carve(int nx_, int ny_, float* q, double* part)
 static double refine_working_set(int nx, int ny) { return 4.0 * (double)refine_floats(nx, ny); }
 
 // The FP32 correction descriptors of one instance: [0] runs vx[0] -> vx[1], [1] back.
-void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, int rows, CorrParams out[CDESC_PER_INST])
+void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, CorrParams out[CDESC_PER_INST])
 {
     const SolveConsts k = solve_consts(a.nx, a.ny, a.dx, a.dy);
     CorrParams cp{};
     cp.nx = a.nx;
     cp.ny = a.ny;
-    cp.seg = std::min(rows > 0 ? rows : 4, a.ny);
-    cp.nstrips = corr_num_strips(a.nx);
-    cp.ntiles = cp.nstrips * ((a.ny + cp.seg - 1) / cp.seg);
-    cp.depth = 1;
     cp.mx = b.mx;
     cp.my = b.my;
     cp.rho = b.rho;
@@ -622,8 +618,6 @@ void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, int row
     cp.max_nxy = (float)k.max_nxy;
     float* const mx[2] = {b.mx, b.mx2};
     float* const my[2] = {b.my, b.my2};
-    // at least 4 rows, as the FP64 wide pass: many instances fill the chip
-    const int rows2 = std::max(corr2_default_rows(a.nx, a.ny), std::min(4, a.ny));
     for (int d = 0; d < 2; ++d) {
         out[d] = cp;
         out[d].vx_a = b.vx[d];
@@ -636,15 +630,6 @@ void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, int row
         out[d].my = my[d];
         out[d].mx_o = mx[1 - d];
         out[d].my_o = my[1 - d];
-        out[2 + d] = out[d];
-        out[2 + d].seg = rows2;
-        out[2 + d].nstrips = corr2_num_strips(a.nx);
-        out[2 + d].ntiles = out[2 + d].nstrips * ((a.ny + rows2 - 1) / rows2);
-        const int rows3 = std::min(a.ny, std::max(a.nx, a.ny) > 256 ? 16 : 8);
-        out[4 + d] = out[d];
-        out[4 + d].seg = rows3;
-        out[4 + d].nstrips = (a.nx - 1 + 57) / 58;
-        out[4 + d].ntiles = out[4 + d].nstrips * ((a.ny + rows3 - 1) / rows3);
     }
 }
 
@@ -742,6 +727,7 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
     const std::vector<RefineBufs>& rb = *env.rb;
     struct Run {
         int id, cur, rebases;
+        int kmax, k;  // sweeps per pass, of this step's
         int64_t n32, n64, ncheck, ndtupdate, checked_at, window, left, wstart;
         double err_k, err_ref, dt_k, ws;
         bool converged;
@@ -888,13 +874,11 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
     std::vector<Run> act;
     size_t q = 0;
     double ws_active = 0.0;
-    WideCorrArgs wa, w2, w3;
+    WideCorrArgs wa;
     std::memset(&wa, 0, sizeof(wa));
-    std::memset(&w2, 0, sizeof(w2));
-    std::memset(&w3, 0, sizeof(w3));
     wa.desc = env.cdesc_dev;
-    w2.desc = env.cdesc_dev;
-    w3.desc = env.cdesc_dev;
+    CorrPlan plan{};
+    bool replan = true;  // the active set has changed
     int rc = SF_OK;
     while (!act.empty() || q < order.size()) {
         while (q < order.size() && (int)act.size() < WIDE_MAX &&
@@ -926,46 +910,39 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
             } else {
                 act.push_back(r);
                 ws_active += r.ws;
+                replan = true;
             }
         }
         if (act.empty()) continue;
-        // three (or two) sweeps per pass for every instance with that many left in its window
-        wa.n_active = 0;
-        w2.n_active = 0;
-        w3.n_active = 0;
-        int tiles = 0, tiles2 = 0, tiles3 = 0;
-        for (size_t k = 0; k < act.size(); ++k) {
-            const size_t base = CDESC_PER_INST * (size_t)act[k].id;
-            if (act[k].left >= 3) {
-                w3.tile_start[w3.n_active] = tiles3;
-                w3.slot_desc[w3.n_active] = (int)base + 4 + act[k].cur;
-                tiles3 += cdesc[base + 4].ntiles;
-                w3.n_active += 1;
-            } else if (act[k].left >= 2) {
-                w2.tile_start[w2.n_active] = tiles2;
-                w2.slot_desc[w2.n_active] = (int)base + 2 + act[k].cur;
-                tiles2 += cdesc[base + 2].ntiles;
-                w2.n_active += 1;
-            } else {
-                wa.tile_start[wa.n_active] = tiles;
-                wa.slot_desc[wa.n_active] = (int)base + act[k].cur;
-                tiles += cdesc[base].ntiles;
-                wa.n_active += 1;
+        if (replan) {
+            int nx[WIDE_MAX], ny[WIDE_MAX], k[WIDE_MAX];
+            for (size_t j = 0; j < act.size(); ++j) {
+                nx[j] = in[act[j].id].nx;
+                ny[j] = in[act[j].id].ny;
             }
+            plan = corr_plan(nx, ny, (int)act.size(), k);
+            for (size_t j = 0; j < act.size(); ++j) act[j].kmax = k[j];
+            replan = false;
         }
+        // one launch: every instance as many sweeps as its plan has and its window leaves
+        int tiles = 0;
+        for (size_t j = 0; j < act.size(); ++j) {
+            Run& r = act[j];
+            r.k = (int)std::min<int64_t>(r.kmax, r.left);
+            wa.tile_start[j] = tiles;
+            wa.slot_desc[j] = CDESC_PER_INST * r.id + r.cur;
+            wa.slot_k[j] = r.k;
+            tiles += corr_plan_tiles(plan, in[r.id].nx, in[r.id].ny, r.k);
+        }
+        wa.n_active = (int)act.size();
         wa.tile_start[wa.n_active] = tiles;
-        w2.tile_start[w2.n_active] = tiles2;
-        w3.tile_start[w3.n_active] = tiles3;
-        if (w3.n_active) HIPCHK(launch_wide_corr3(w3, s));
-        if (w2.n_active) HIPCHK(launch_wide_corr2(w2, s));
-        if (wa.n_active) HIPCHK(launch_wide_corr(wa, s));
+        HIPCHK(launch_wide_corr(wa, plan, s));
         std::vector<Run> keep;
         keep.reserve(act.size());
         for (Run& r : act) {
-            const int64_t adv = r.left >= 3 ? 3 : (r.left >= 2 ? 2 : 1);
             r.cur ^= 1;
-            r.n32 += adv;
-            r.left -= adv;
+            r.n32 += r.k;
+            r.left -= r.k;
             bool done = false;
             if (r.left == 0) {
                 rc = end_window(r);
@@ -981,6 +958,7 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
                 keep.push_back(r);
             }
         }
+        replan = keep.size() != act.size();
         act.swap(keep);
     }
     HIPCHK(hipStreamSynchronize(s));
@@ -1071,7 +1049,7 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         for (int i = 0; i < n; ++i) {
             rb[(size_t)i] = refine_carve(in[i].nx, in[i].ny, c->b_pool32 + foff[(size_t)i],
                                          c->b_part + (size_t)3 * RED_MAX_BLOCKS * i);
-            refine_descriptors(in[i], rb[(size_t)i], prm ? prm->rows : 0, &cdesc[CDESC_PER_INST * (size_t)i]);
+            refine_descriptors(in[i], rb[(size_t)i], &cdesc[CDESC_PER_INST * (size_t)i]);
         }
         HIPCHK(hipMemcpyAsync(c->b_cdesc, cdesc.data(), sizeof(CorrParams) * CDESC_PER_INST * (size_t)n,
                               hipMemcpyHostToDevice, s));

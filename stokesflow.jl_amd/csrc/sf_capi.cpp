@@ -266,7 +266,7 @@ int PassTimer::begin(hipStream_t s, int precision, int k)
     const int slot = (head + count) % RING;
     for (int q = 0; q < 2; ++q)
         if (!ev[2 * slot + q]) HIPCHK(hipEventCreate(&ev[2 * slot + q]));
-    kind[slot] = (precision ? 8 : 0) + std::min(std::max(k, 0), 7);
+    kind[slot] = (precision ? 16 : 0) + std::min(std::max(k, 0), 15);
     HIPCHK(hipEventRecord(ev[2 * slot], s));
     return SF_OK;
 }
@@ -341,7 +341,7 @@ extern "C" int sf_ctx_pass_times(sf_ctx* c, sf_pass_time* out, int cap, int* n_o
     int m = 0;
     for (int q = 0; q < PassTimer::KINDS; ++q) {
         if (!c->timer.n[q]) continue;
-        if (m < cap) out[m] = sf_pass_time{q >= 8 ? 1 : 0, q % 8, c->timer.n[q], c->timer.sec[q]};
+        if (m < cap) out[m] = sf_pass_time{q / 16, q % 16, c->timer.n[q], c->timer.sec[q]};
         ++m;
     }
     if (n_out) *n_out = m;
@@ -1339,6 +1339,10 @@ extern "C" int sf_solve_stokes_refined(sf_ctx* c, double* P, double* Vx_pad, dou
     const bool corr_pairs = c->fuse != 1;
     // sweeps per pass: the context's setting, or the size default of the FP32 sweeps
     const int corr_k = c->fuse == 0 ? corr_default_fusion(nx, ny) : c->fuse;
+    // with neither passes nor tile rows set: the resident passes of the size default
+    const bool resident = c->fuse == 0 && c->pair_rows == 0;
+    int plan_k = 0;
+    const CorrPlan plan = corr_plan(&nx, &ny, 1, &plan_k);
     if (corr_pairs) {
         rc = refine_reserve_m2(c);
         if (rc) return rc;
@@ -1444,6 +1448,25 @@ extern "C" int sf_solve_stokes_refined(sf_ctx* c, double* P, double* Vx_pad, dou
         steps = std::min(steps, ncheck - n32 % ncheck);
         if (use_fss) steps = std::min(steps, ndtupdate - n32 % ndtupdate);
         int64_t it = 0;
+        while (resident && it < steps) {
+            const int kk = (int)std::min<int64_t>(plan_k, steps - it);
+            cp.vx_a = c->r_vx[cur];
+            cp.vy_a = c->r_vy[cur];
+            cp.p_a = c->r_p[cur];
+            cp.vx_b = c->r_vx[1 - cur];
+            cp.vy_b = c->r_vy[1 - cur];
+            cp.p_b = c->r_p[1 - cur];
+            cp.mx = c->r_mx;
+            cp.my = c->r_my;
+            cp.mx_o = c->r_mx2;
+            cp.my_o = c->r_my2;
+            rc = timed_corr(kk, [&] { return launch_corr_resident(cp, kk, plan.r, plan.waves, s); });
+            if (rc) return rc;
+            cur = 1 - cur;
+            std::swap(c->r_mx, c->r_mx2);
+            std::swap(c->r_my, c->r_my2);
+            it += kk;
+        }
         for (; corr_k >= 3 && it + corr_k <= steps; it += corr_k) {
             cp.vx_a = c->r_vx[cur];
             cp.vy_a = c->r_vy[cur];

@@ -282,7 +282,7 @@ extern "C" int sf_ensemble_create(sf_ctx* c, const sf_step_args* members, int n,
         for (int i = 0; i < n; ++i) {
             e->rb[(size_t)i] = refine_carve(members[i].nx, members[i].ny, e->pool32 + foff[(size_t)i],
                                             e->rpart + (size_t)3 * RED_MAX_BLOCKS * i);
-            refine_descriptors(bi[(size_t)i], e->rb[(size_t)i], prm ? prm->rows : 0, &e->cdesc[CDESC_PER_INST * (size_t)i]);
+            refine_descriptors(bi[(size_t)i], e->rb[(size_t)i], &e->cdesc[CDESC_PER_INST * (size_t)i]);
         }
         er = hipMemcpyAsync(e->cdesc_dev, e->cdesc.data(), sizeof(CorrParams) * CDESC_PER_INST * (size_t)n, hipMemcpyHostToDevice,
                             e->stream);

@@ -99,7 +99,7 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n, const
                    const std::vector<int>& order, double budget, int depth, std::vector<BatchResult>& res);
 size_t refine_floats(int nx, int ny);
 RefineBufs refine_carve(int nx, int ny, float* q, double* part);
-void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, int rows, CorrParams out[CDESC_PER_INST]);
+void refine_descriptors(const sf_batch_instance& a, const RefineBufs& b, CorrParams out[CDESC_PER_INST]);
 int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, int n,
                            const std::vector<BatchInstance>& desc, std::vector<CorrParams>& cdesc,
                            const std::vector<int>& order, double budget, std::vector<BatchResult>& res);
@@ -125,7 +125,7 @@ struct PTBuffers {
 // in a ring and resolved lazily (a slot is resolved when the ring wraps, long after its launch
 // ended), summed per (precision, iterations per launch).  Instrumentation only.
 struct PassTimer {
-    enum { RING = 256, KINDS = 16 };
+    enum { RING = 256, KINDS = 32 };
     bool on = false;
     hipEvent_t ev[2 * RING] = {};
     int kind[RING] = {};

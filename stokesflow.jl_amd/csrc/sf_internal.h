@@ -165,6 +165,15 @@ hipError_t launch_pt_corr(const CorrParams& p, bool check, hipStream_t s);
 hipError_t launch_pt_corr2(const CorrParams& p, hipStream_t s);
 // k = 3 or 4 correction sweeps per pass (corrk_tile<k>, 64 - 2k output columns per strip).
 hipError_t launch_pt_corrk(const CorrParams& p, int k, hipStream_t s);
+// k sweeps per pass on tiles of waves * r rows held in registers (sf_ctr_tile.h).
+hipError_t launch_corr_resident(const CorrParams& p, int k, int r, int waves, hipStream_t s);
+// The size default: the shape for a set of grids and per grid the sweeps of a pass.
+#define CORR_MAX_K 12
+struct CorrPlan {
+    int r, waves;
+};
+CorrPlan corr_plan(const int* nx, const int* ny, int n, int* k);
+int corr_plan_tiles(const CorrPlan& plan, int nx, int ny, int k);
 hipError_t launch_resid_f64(const ResidParams& p, int nb, hipStream_t s);
 hipError_t launch_update_f64(double* a, const float* d, int64_t n, hipStream_t s);
 hipError_t launch_cast_f32(float* dst, const double* src, int64_t n, hipStream_t s);
@@ -276,23 +285,20 @@ WidePlan wide_plan(const int* nx, const int* ny, int n, int* k, int* rows);
 int wide_resident_tiles(const WidePlan& plan, int nx, int ny, int k);
 hipError_t launch_wide_resident(const WideArgs& a, const WidePlan& plan, hipStream_t s);
 
-// Wide mode of the FP32 correction sweeps: slot k runs descriptor slot_desc[k] (two
+// Wide mode of the FP32 correction sweeps: slot i runs slot_k[i] sweeps on descriptor slot_desc[i] (two
 // descriptors per instance, one per ping-pong direction).
 struct WideCorrArgs {
     const CorrParams* desc;
     int n_active;
     int tile_start[WIDE_MAX + 1];
     int slot_desc[WIDE_MAX];
+    int slot_k[WIDE_MAX];
 };
-hipError_t launch_wide_corr(const WideCorrArgs& a, hipStream_t s);
-hipError_t launch_wide_corr2(const WideCorrArgs& a, hipStream_t s);  // two sweeps per slot
-hipError_t launch_wide_corr3(const WideCorrArgs& a, hipStream_t s);  // three sweeps per slot
-int corr_num_strips(int nx);
-int corr2_num_strips(int nx);
+hipError_t launch_wide_corr(const WideCorrArgs& a, const CorrPlan& plan, hipStream_t s);
 int corr2_default_rows(int nx, int ny);
-// Correction descriptors per instance in the wide refined mode: [parity] one sweep,
-// [2 + parity] two sweeps, [4 + parity] three; the state and the momentum ping-pong together.
-#define CDESC_PER_INST 6
+// Correction descriptors per instance in the wide refined mode, by parity: the state and the
+// momentum ping-pong together.
+#define CDESC_PER_INST 2
 
 hipError_t launch_batch_solve(const BatchInstance* inst, const int* order, int n_inst, int* queue,
                               BatchResult* res, int threads, int nblocks, hipStream_t s);

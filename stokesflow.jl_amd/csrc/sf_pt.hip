@@ -302,7 +302,7 @@ hipError_t launch_pt_pair(const PTParams& p0, hipStream_t s)
 // / 2.79.  Four iterations per pass from 449 nodes per side, two below.
 int pt_default_fusion(int nx, int ny) { return std::max(nx, ny) > 448 ? 4 : 2; }
 
-// Sweeps per pass of the FP32 correction solver when the context leaves it open (three from 769
+// Sweeps per one-wave pass of the FP32 correction solver when only the tile rows are given (three from 769
 // nodes per side; us per sweep, K=3 against K=2: 1024^2 7.82 (8-row tiles) against 8.8, 1280^2
 // 9.54 against 11.2, 1536^2 12.45 against 14.45).  Above 1536, four (interleaved repetitions on
 // one box, us per sweep, four against three: 4096^2 79.5 against 87.7, 3072^2 44.9 against 53.7,

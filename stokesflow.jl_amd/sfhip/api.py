@@ -166,10 +166,10 @@ def pass_times(nx, ny):
     """Totals of the timed pass launches of the nx x ny context (sf_ctx_pass_times): a list of
     dicts with precision (0 FP64, 1 FP32), iters_per_launch, launches and seconds."""
     ctx = context(nx, ny)
-    buf = (_lib.PassTime * 16)()
+    buf = (_lib.PassTime * 32)()
     n = C.c_int(0)
-    check(ctx.lib.sf_ctx_pass_times(ctx.handle, buf, 16, C.byref(n)))
-    return [buf[i].as_dict() for i in range(min(n.value, 16))]
+    check(ctx.lib.sf_ctx_pass_times(ctx.handle, buf, 32, C.byref(n)))
+    return [buf[i].as_dict() for i in range(min(n.value, 32))]
 
 
 def set_pt_tuning(nx, ny, rows=0, depth=0, max_waves=-1):
@@ -286,7 +286,7 @@ def solveStokes_batched(problems, *, mode="auto", rows=0, depth=0, threads=0, ma
     pass, 1 to 3; default by size).
     ``mixed_precision=True`` (wide mode): every instance is solved as
     ``solveStokes(..., mixed_precision=True)`` solves it (FP32 sweeps inside FP64 defect
-    correction), one to three FP32 sweeps per launch of all active instances.
+    correction), several FP32 sweeps per launch of all active instances.
     """
     n = len(problems)
     arr = _batch_instances(problems)

@@ -429,3 +429,28 @@ def test_autotune_keeps_results(gpu, golden):
 def test_dram_probe(gpu):
     r = sfhip.probe_dram(1 << 26)
     assert 500.0 < r["copy_gbs"] < 9000.0 and 500.0 < r["r3w1_gbs"] < 9000.0
+
+
+@pytest.mark.parametrize("nx,ny,cap,rebase", [(3, 3, 40, 0), (65, 63, 331, 0), (300, 257, 90, 31), (512, 500, 60, 0), (1000, 777, 47, 0),
+                                              (1201, 1024, 26, 0)])
+def test_refined_default_passes_bitwise(gpu, nx, ny, cap, rebase):
+    """The size default's passes, whole and cut short by the windows, against one sweep per launch."""
+    S = cases.smooth_state(nx, ny, seed=nx)
+    out = []
+    for fuse in (1, 0):
+        G = to_gpu(S, list(S.keys()))
+        st = {}
+        try:
+            sfhip.set_pt_fusion(nx, ny, fuse, 0)
+            sfhip.solveStokes(G["P"], G["Vx_pad"], G["Vy_pad"], G["rho_vy"], G["mu_b"], G["mu_p"], None, None, None,
+                              None, None, None, None, G["dVx"], G["dVy"], None, None, G["Vx_s"], G["Vy_s"], 1.0,
+                              1.0 / (nx - 1), 1.0 / (ny - 1), nx, ny, 0.0, 0.5, eps=1e-12, print_info=False, iterMax=cap,
+                              stats=st, mixed_precision=True, refine={"rebase_interval": rebase})
+        finally:
+            sfhip.set_pt_fusion(nx, ny, 0, 0)
+        torch.cuda.synchronize()
+        out.append((st, {k: sfhip.to_numpy(G[k]) for k in ("Vx_pad", "Vy_pad", "P", "dVx", "dVy")}))
+    (s1, a1), (s2, a2) = out
+    assert s1["n_fp32_iter"] == s2["n_fp32_iter"]
+    for k in a1:
+        assert np.array_equal(a1[k], a2[k], equal_nan=True), k
