@@ -9,12 +9,14 @@ using namespace sf;
 namespace sf {
 
 // Grid mode: what a pass costs besides its iterations, us: the barrier, and the tile read again past
-// caches that the barrier has emptied.  (384x300 takes 2.58 us per iteration planned with 4, 2.46 with 8;
-// 97x130 2.04 with 8, 2.10 with 11.)
+// caches that the barrier has emptied.
 #define GRID_PASS_US 8.0
-// and the grids that resident passes are for: 1000x777 takes 7.7 us per iteration with them and 9.6
-// with one-wave passes of three, 1024^2 11.3 and 10.9, larger ones the same within 7% (64^2 1.83 and 3.48,
-// 301x257 2.34 and 4.09, 512^2 3.55 and 8.04).
+// The same where every tile stays in registers: the exchange with the tiles around (600x520 takes 2.30 us
+// per iteration planned with 3.5, 2.65 with 4.5; 64^2 1.34 with both, 1.46 with 6).
+#define GRID_KEPT_US 3.5
+// The grids that resident passes are for (us per iteration, and with one-wave passes of three): 64^2 1.34,
+// 3.48; 301x257 1.56, 4.09; 384x300 1.62, 6.49; 512^2 2.13, 8.04; 730^2 4.0, 10.6; past what the chip holds
+// at once 1000x777 8.3, 9.6; 1024^2 11.3, 10.9, and larger ones the same within 7%.
 #define GRID_RESIDENT_NODES 900000
 
 // Per-instance scratch (doubles) of the batched solver: ping-pong state, tau/divV, Rx/Ry, scalars.
@@ -194,7 +196,7 @@ GridShape grid_launch_shape(const BatchInstance& d, int k)
 {
     if (k == 0) {
         double us;
-        const PTPlan plan = pt_plan_resident(d.nx, d.ny, GRID_RESIDENT_MAX_K, GRID_PASS_US, &us);
+        const PTPlan plan = pt_plan_resident(d.nx, d.ny, GRID_RESIDENT_MAX_K, GRID_PASS_US, GRID_KEPT_US, &us);
         if (plan.kind == PT_PLAN_RESIDENT && (int64_t)d.nx * d.ny <= GRID_RESIDENT_NODES) {
             const int out = 64 - 2 * plan.k, seg = plan.waves * plan.r - 2 * plan.k;
             const int64_t t = (int64_t)((d.nx - 1 + out - 1) / out) * ((d.ny + seg - 1) / seg);
@@ -228,8 +230,15 @@ extern "C" int sf_set_grid_wait_limit(double seconds)
 namespace sf {
 
 // Grid mode: the barrier words and the partials of the context.
-static int grid_reserve(sf_ctx* c, int n)
+static int grid_reserve(sf_ctx* c, int n, size_t exch)
 {
+    if (exch > c->g_exch_cap) {
+        if (c->g_exch) HIPCHK(hipFree(c->g_exch));
+        c->g_exch = nullptr;
+        c->g_exch_cap = 0;
+        HIPCHK(dalloc(&c->g_exch, exch));
+        c->g_exch_cap = exch;
+    }
     if (!c->g_part) HIPCHK(dalloc(&c->g_part, 3 * (size_t)GRID_MAX_WAVES));
     if (n > c->g_cap) {
         if (c->g_sync) HIPCHK(hipFree(c->g_sync));
@@ -1063,17 +1072,23 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         HIPCHK(hipStreamSynchronize(s));
     } else if (mode == SF_BATCH_GRID) {
         // one instance after another, each solved by one launch over the whole chip
-        rc = grid_reserve(c, n);
-        if (rc) return rc;
         const int k = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 0;
+        std::vector<GridShape> shape((size_t)n);
+        size_t exch = 0;
+        for (int i = 0; i < n; ++i) {
+            shape[(size_t)i] = grid_launch_shape(host[(size_t)i], k);
+            if (shape[(size_t)i].r) exch = std::max(exch, grid_exchange_doubles(in[i].nx, in[i].ny));
+        }
+        rc = grid_reserve(c, n, exch);
+        if (rc) return rc;
         HIPCHK(hipMemsetAsync(c->g_sync, 0, sizeof(unsigned long long) * GRID_SYNC_WORDS * (size_t)n, s));
         const double wait_s = grid_wait_seconds();
         const uint64_t wait_ticks = grid_wait_limit();
         for (int qi = 0; qi < n; ++qi) {
             const int i = order[(size_t)qi];
-            const GridShape gs = grid_launch_shape(host[(size_t)i], k);
+            const GridShape& gs = shape[(size_t)i];
             const GridArgs ga{c->b_inst + i, c->b_res + i, c->g_sync + (size_t)GRID_SYNC_WORDS * i, c->g_part,
-                              gs.nwg, gs.waves, gs.k, gs.r, wait_ticks};
+                              gs.nwg, gs.waves, gs.k, gs.r, wait_ticks, c->g_exch};
             HIPCHK(launch_grid_solve(ga, s));
         }
         std::vector<unsigned long long> sync((size_t)GRID_SYNC_WORDS * n);

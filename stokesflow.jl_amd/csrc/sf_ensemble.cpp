@@ -31,6 +31,7 @@ struct sf_ensemble {
     unsigned long long* gsync = nullptr;  // grid mode: GRID_SYNC_WORDS barrier words per member
     unsigned long long* hsync = nullptr;  // pinned
     double* gpart = nullptr;              // grid mode: 3 * GRID_MAX_WAVES partials
+    double* gexch = nullptr;              // grid mode: exchange of the resident passes, members in turn
     std::vector<GridShape> gshape;        // grid mode: each member's launch
     hipGraph_t graph[2] = {nullptr, nullptr};  // persistent: [0] whole step; wide: [0] marker -> grid, [1] RK4
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -57,7 +58,7 @@ static void free_ensemble(sf_ensemble* e)
     }
     for (void* p : {(void*)e->pool, (void*)e->inst, (void*)e->order_dev, (void*)e->queue, (void*)e->res,
                     (void*)e->cnt, (void*)e->part, (void*)e->pool32, (void*)e->rpart, (void*)e->cdesc_dev,
-                    (void*)e->gsync, (void*)e->gpart})
+                    (void*)e->gsync, (void*)e->gpart, (void*)e->gexch})
         if (p) (void)hipFree(p);
     for (void* p : {(void*)e->hcnt, (void*)e->hres, (void*)e->hscal, (void*)e->hpart, (void*)e->hdt, (void*)e->hsync})
         if (p) (void)hipHostFree(p);
@@ -125,7 +126,7 @@ static hipError_t ensemble_enqueue_persistent(sf_ensemble* e)
             const int i = e->order[(size_t)q];
             const GridShape& gs = e->gshape[(size_t)i];
             const GridArgs ga{e->inst + i, e->res + i, e->gsync + (size_t)GRID_SYNC_WORDS * i, e->gpart, gs.nwg, gs.waves,
-                              gs.k, gs.r, grid_wait_limit()};
+                              gs.k, gs.r, grid_wait_limit(), e->gexch};
             r = launch_grid_solve(ga, e->stream);
         }
     } else {
@@ -257,7 +258,15 @@ extern "C" int sf_ensemble_create(sf_ctx* c, const sf_step_args* members, int n,
     e->order = batch_order(dims);
     if (e->grid) {
         e->gshape.resize((size_t)n);
-        for (int i = 0; i < n; ++i) e->gshape[(size_t)i] = grid_launch_shape(e->desc[(size_t)i], e->gk);
+        size_t exch = 0;
+        for (int i = 0; i < n; ++i) {
+            e->gshape[(size_t)i] = grid_launch_shape(e->desc[(size_t)i], e->gk);
+            if (e->gshape[(size_t)i].r) exch = std::max(exch, grid_exchange_doubles(members[i].nx, members[i].ny));
+        }
+        if (exch && (er = dalloc(&e->gexch, exch)) != hipSuccess) {
+            free_ensemble(e);
+            return set_err(SF_ERR_HIP, "%s: %s", who, hipGetErrorString(er));
+        }
     }
     e->nblocks = batch_grid(c, n, threads, prm ? prm->max_blocks : 0);
     if (e->refined) {

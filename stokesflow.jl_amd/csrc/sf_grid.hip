@@ -5,9 +5,11 @@
 // launch of at most one workgroup per CU walks the same pass schedule as sf_solve_stokes (passes of
 // several PT iterations, the single iterations at checks, dt refreshes and iterMax), and a grid barrier
 // separates the passes.  Small and middle grids take passes of up to GRID_RESIDENT_MAX_K iterations on
-// tiles in registers, a tile per workgroup of up to 16 waves: the barrier, and the tile that every pass
-// reads past caches the barrier has emptied, cost about 8 us and are paid once per 5 to 14 iterations
-// (384x300: 2.46 us per iteration; 6.5 with passes of three).  Larger grids take passes of up to three on
+// tiles in registers, a tile per workgroup of up to 16 waves.  Where the chip holds all tiles at once they
+// stay there from pass to pass, and only the nodes that other tiles need go through memory, each tile
+// waiting for its neighbours alone (GridExchange: 384x300 takes 1.62 us per iteration; 2.46 where every
+// pass met at the barrier and read its tile again, which costs 8 us, and 6.5 with passes of three).
+// Larger grids take passes of up to three on
 // tiles of one wave, one to eight waves per workgroup.  Tiles go out t = band, band + G, ... (the
 // workgroups of one XCD hold consecutive bands).  The dt refresh and the err check
 // reduce over the whole grid in two steps (a partial per wave, then every wave sums the partials
@@ -213,6 +215,58 @@ __device__ inline void grid_copy(double* __restrict__ dst, const double* __restr
 
 }  // namespace
 
+// Between passes on a tile that stays in registers: the nodes that other tiles need go through memory,
+// by agent-scope stores and loads, which pass the XCDs' L2 (two buffers in turn; a tile may write a buffer
+// again once its neighbours have finished the pass after the one that read it, which their flags say).
+// No cache is written back or emptied, and a tile waits only for those within its reach.
+struct GridExchange {
+    static constexpr bool RUN = true;
+    int passes;
+    u64* flags;
+    double* buf;
+    int64_t n;       // nodes of a field
+    int nx1;         // columns
+    u64 seq;         // passes that every tile has posted in this launch
+    u64* s;          // sync words
+    uint64_t limit;
+    int strip, segid, nstrips, nseg, reach;  // reach: segments above and below that the tile reads
+
+    __device__ void put(int r, int c, double a, double b, double d, double e, double f) const
+    {
+        double* const q = buf + (seq & 1) * 5 * n + (int64_t)r * nx1 + c;
+        __hip_atomic_store(q, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(q + n, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(q + 2 * n, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(q + 3 * n, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(q + 4 * n, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ void get(int r, int c, double& a, double& b, double& d, double& e, double& f) const
+    {
+        const double* const q = buf + ((seq - 1) & 1) * 5 * n + (int64_t)r * nx1 + c;
+        a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        b = __hip_atomic_load(q + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        d = __hip_atomic_load(q + 2 * n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        e = __hip_atomic_load(q + 3 * n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        f = __hip_atomic_load(q + 4 * n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ bool swap()
+    {
+        ++seq;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have reached memory
+        __syncthreads();
+        int ok = 1;
+        if (threadIdx.x < SF_WAVE) {
+            if (threadIdx.x == 0)
+                __hip_atomic_store(flags + 16 * (segid * nstrips + strip), seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int ds = (int)threadIdx.x % 3 - 1, dg = (int)threadIdx.x / 3 - reach;
+            const int ns = strip + ds, ng = segid + dg;
+            if (dg <= reach && ns >= 0 && ns < nstrips && ng >= 0 && ng < nseg)
+                ok = wait_agent(flags + 16 * (ng * nstrips + ns), seq, s, limit);
+        }
+        return __syncthreads_or(!ok) == 0;
+    }
+};
+
 // R = 0: one-wave passes of K iterations, 1 to 3 (the four-iteration tile spills beside the loop
 // control).  R > 0: passes of up to K = a.k iterations on tiles of R rows per wave held in registers, a
 // workgroup per tile.
@@ -265,6 +319,15 @@ __global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) voi
 
     __shared__ double lds[R ? PTR_LDS(GRID_RESIDENT_WAVES) : 1];
     const int band = __builtin_amdgcn_readfirstlane(bar.band), waves = blockDim.x >> 6;
+    GridExchange ex{1, (u64*)a.exch, a.exch + GRID_FLAG_WORDS, (int64_t)(nx - 1) * ny, nx - 1, 0ull, a.sync, a.limit, 0, 0, 1, 1, 1};
+    bool kept = false;  // the tiles of the full passes are all resident
+    if constexpr (R > 0) {
+        const int out = SF_WAVE - 2 * a.k, seg = waves * R - 2 * a.k;
+        ex.nstrips = (nx - 1 + out - 1) / out;
+        ex.nseg = (ny + seg - 1) / seg;
+        ex.reach = (a.k + seg - 1) / seg;
+        kept = ex.nstrips * ex.nseg <= min((int)gridDim.x, GRID_FLAGS) && 3 * (2 * ex.reach + 1) <= SF_WAVE;
+    }
     double err = 2.0 * eps;
     int64_t iter = 1;
     int pf = 0;  // passes so far, mod 2: the state (V, P, dV) is in the caller's buffers when 0
@@ -274,10 +337,13 @@ __global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) voi
         // one-wave passes have k = K, and where K do not fit, single iterations follow (the same
         // bits); resident passes take as many as fit
         int k = K;
+        int64_t passes = 1;
         if constexpr (R > 0) {
             int64_t fit = ncheck - 1 - (iter - 1) % ncheck;
             if (fss) fit = min(fit, ndtupdate - (iter - 1) % ndtupdate);
-            k = (int)min((int64_t)a.k, min(fit, iter_max - iter));
+            fit = min(fit, iter_max - iter);
+            k = (int)min((int64_t)a.k, fit);
+            if (kept && k == a.k) passes = fit / k;  // all of them on tiles kept in registers
         }
         bool fused = R > 0 ? k > 0 : K > 1 && iter + K - 1 < iter_max;
         if constexpr (R == 0)
@@ -290,7 +356,12 @@ __global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) voi
             if constexpr (R > 0) {
                 const int out = SF_WAVE - 2 * k, seg = waves * R - 2 * k;
                 const int nstrips = (nx - 1 + out - 1) / out, ntiles = nstrips * ((ny + seg - 1) / seg);
-                for (int t = band; t < ntiles; t += gridDim.x) ptr_tile<R>(pp, k, seg, t % nstrips, t / nstrips, lds);
+                for (int t = band; t < ntiles; t += gridDim.x) {
+                    ex.passes = (int)passes;
+                    ex.strip = t % nstrips;
+                    ex.segid = t / nstrips;
+                    if (!ptr_tile<R>(pp, k, seg, ex.strip, ex.segid, lds, ex)) return;
+                }
             } else {
                 const int ntiles = pp.ntiles, nstrips = pp.nstrips;
                 if constexpr (K == 3) {
@@ -301,13 +372,13 @@ __global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) voi
             }
             pf ^= 1;
             if (!bar.sync()) return;
-            if (fss && (iter + k - 1) % ndtupdate == 0) {
+            if (fss && (iter + passes * k - 1) % ndtupdate == 0) {
                 double dtc;
                 if (!grid_dt(pp.vx_b, pp.vy_b, &dtc)) return;
                 if (blockIdx.x == 0 && threadIdx.x == 0) I.scal[SC_DT] = dtc;
                 if (!bar.sync()) return;
             }
-            iter += k;
+            iter += passes * k;
             continue;
         }
         const PTParams GRID_CONST& pp = I.wpt[pf];
@@ -392,8 +463,9 @@ __global__ __launch_bounds__(64 * (R ? GRID_RESIDENT_WAVES : GRID_WG_WAVES)) voi
 }
 
 // Every word but the sticky failure flag, which only the host clears.
-__global__ void grid_zero_sync(unsigned long long* p)
+__global__ void grid_zero_sync(unsigned long long* p, unsigned long long* flags)
 {
+    for (int k = threadIdx.x; flags && k < GRID_FLAGS; k += blockDim.x) flags[16 * k] = 0ull;
     for (int k = threadIdx.x; k < GRID_SYNC_WORDS; k += blockDim.x)
         if (k != GRID_SYNC_STICKY) p[k] = 0ull;
 }
@@ -449,8 +521,8 @@ double grid_wait_seconds() { return grid_wait_s.load(); }
 
 hipError_t launch_grid_solve(const GridArgs& a, hipStream_t s)
 {
-    if (a.nwg < 1 || a.nwg > grid_capacity(a.k, a.r, a.wg_waves)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(grid_zero_sync, dim3(1), dim3(256), 0, s, a.sync);
+    if (a.nwg < 1 || a.nwg > grid_capacity(a.k, a.r, a.wg_waves) || (a.r && !a.exch)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(grid_zero_sync, dim3(1), dim3(256), 0, s, a.sync, a.r ? (unsigned long long*)a.exch : nullptr);
     GridArgs arg = a;
     void* args[] = {&arg};
     return hipLaunchKernel(grid_kernel(a.k, a.r), dim3(a.nwg), dim3(64 * a.wg_waves), args, 0, s);

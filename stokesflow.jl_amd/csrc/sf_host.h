@@ -274,4 +274,6 @@ struct sf_ctx {
     unsigned long long* g_sync = nullptr;  // GRID_SYNC_WORDS barrier words per instance
     int g_cap = 0;
     double* g_part = nullptr;  // 3 * GRID_MAX_WAVES partials
+    double* g_exch = nullptr;  // exchange of the resident passes (GridArgs), shared by the instances in turn
+    size_t g_exch_cap = 0;
 };

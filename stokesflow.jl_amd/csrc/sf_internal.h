@@ -93,8 +93,9 @@ struct PTPlan {
     int r, waves;  // resident: rows per wave, waves
 };
 PTPlan pt_plan(int nx, int ny);
-// The best resident shape with passes launch_us apart, and its modelled time per iteration.
-PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double* us_per_iter);
+// The best resident shape with passes launch_us apart, and its modelled time per iteration; kept_us: the
+// time between passes of tiles that stay in registers, where all are resident at once (0: they do not).
+PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double kept_us, double* us_per_iter);
 hipError_t launch_pt_plan(const PTParams& p, const PTPlan& plan, int k, hipStream_t s);
 // Snapshot staging: dst = (float)(src + shift) (sf_snapshot.hip).
 hipError_t launch_snap_cast(const double* src, float* dst, int64_t n, double shift, hipStream_t s);
@@ -241,7 +242,11 @@ struct GridArgs {
     int nwg, wg_waves;
     int k, r;        // PT iterations per pass; rows per wave of the resident passes, 0: one-wave passes, k <= 3
     uint64_t limit;  // wall-clock ticks a workgroup may wait at a barrier
+    double* exch;    // resident passes: GRID_FLAG_WORDS flags, then grid_exchange_doubles of exchanged nodes
 };
+#define GRID_FLAGS 256  // tiles that may stay in registers, a 128-byte line each
+#define GRID_FLAG_WORDS (16 * GRID_FLAGS)
+inline size_t grid_exchange_doubles(int nx, int ny) { return GRID_FLAG_WORDS + (size_t)10 * (nx - 1) * ny; }
 // k = PT iterations per pass (1, 2 or 3; four need more than 256 VGPRs in this kernel); waves =
 // waves per workgroup (1 to GRID_WG_WAVES).
 int grid_capacity(int k, int r, int waves);

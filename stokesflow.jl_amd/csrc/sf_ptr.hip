@@ -15,7 +15,8 @@ __global__ __launch_bounds__(64 * PTR_MAX_WAVES) void ptr_tile_f64(PTParams p, i
     __shared__ double lds[PTR_LDS(PTR_MAX_WAVES)];
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int nstrips = p.nstrips;
-    ptr_tile<R>(p, k, p.seg, logical % nstrips, logical / nstrips, lds);
+    PTROnce once;
+    ptr_tile<R>(p, k, p.seg, logical % nstrips, logical / nstrips, lds, once);
 }
 
 hipError_t launch_pt_resident(const PTParams& p0, int k, int r, int waves, hipStream_t s)
@@ -70,7 +71,7 @@ static int64_t resident_tiles(int nx, int ny, int rows, int k)
 // Measured against the passes before (us per iteration): 64^2 1.30 (2.6), 301x257 1.64 (3.1), 512^2 2.6
 // (4.65), 700^2 3.85 (about 6.5) resident; 1024^2 6.3 (9.1), 2048^2 19.4 (29.4), 4096^2 69.7 (112)
 // pipelined.  They cross near 730^2: resident 800^2 5.3 against 4.7, pipelined 600^2 3.6 against 2.95.
-PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double* us_per_iter)
+PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double kept_us, double* us_per_iter)
 {
     const int cus = 256;
     PTPlan best{};
@@ -81,7 +82,8 @@ PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double* us_p
                 const int64_t wgs = resident_tiles(nx, ny, sh.waves * sh.r, k);
                 const double rounds = (double)((wgs + cus - 1) / cus);
                 const double fixed = sh.fixed * (1.0 + 0.5 * std::min(1.0, (double)wgs / cus));
-                const double us = (launch_us + rounds * (fixed + k * sh.iter)) / k;
+                double us = (launch_us + rounds * (fixed + k * sh.iter)) / k;
+                if (kept_us > 0.0 && wgs <= cus) us = (kept_us + k * sh.iter) / k;
                 if (us < best_us) {
                     best_us = us;
                     best = PTPlan{PT_PLAN_RESIDENT, k, 0, sh.r, sh.waves};
@@ -95,7 +97,7 @@ PTPlan pt_plan(int nx, int ny)
 {
     const int cus = 256;
     double best_us;
-    PTPlan best = pt_plan_resident(nx, ny, PT_PLAN_MAX_K, 2.5, &best_us);
+    PTPlan best = pt_plan_resident(nx, ny, PT_PLAN_MAX_K, 2.5, 0.0, &best_us);
     const int k = PT_PLAN_MAX_K, lag = 9;
     const int strips = (nx - 1 + SF_WAVE - 2 * k - 1) / (SF_WAVE - 2 * k);
     for (int nseg = 1; nseg <= ny && (int64_t)strips * (nseg - 1) < 12 * cus; ++nseg) {
@@ -202,7 +204,8 @@ __global__ __launch_bounds__(64 * PTR_MAX_WAVES) void wide_ptr_kernel(WideArgs a
     const int k = a.slot_pf[i] >> 1;
     const auto& pp = ((WideInstC*)a.desc)[a.slot_inst[i]].wpt[a.slot_pf[i] & 1];
     const int out = SF_WAVE - 2 * k, nstrips = (pp.nx - 1 + out - 1) / out;
-    ptr_tile<R>(pp, k, (int)(blockDim.x >> 6) * R - 2 * k, t % nstrips, t / nstrips, lds);
+    PTROnce once;
+    ptr_tile<R>(pp, k, (int)(blockDim.x >> 6) * R - 2 * k, t % nstrips, t / nstrips, lds, once);
 }
 
 int wide_resident_tiles(const WidePlan& plan, int nx, int ny, int k)

@@ -52,8 +52,20 @@ __device__ __forceinline__ PTRCell ptr_cell(const PTPConst& k, double vx, double
     return o;
 }
 
-template <int R, class PP>
-__device__ __forceinline__ void ptr_tile(const PP& p, int K, int seg, int strip, int segid, double* lds)
+// No exchange: one pass.
+struct PTROnce {
+    static constexpr bool RUN = false;
+    int passes = 1;
+    __device__ void put(int, int, double, double, double, double, double) const {}
+    __device__ void get(int, int, double&, double&, double&, double&, double&) const {}
+    __device__ bool swap() { return true; }
+};
+
+// ex: what happens between passes where the caller runs several on the same tile (ex.passes of them): the
+// inner nodes stay in registers, those within K of another tile go out (put), the waves meet and
+// wait for the other tiles (swap; false ends the run), and the outer nodes come in (get).
+template <int R, class PP, class EX>
+__device__ __forceinline__ bool ptr_tile(const PP& p, int K, int seg, int strip, int segid, double* lds, EX& ex)
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -136,102 +148,125 @@ __device__ __forceinline__ void ptr_tile(const PP& p, int K, int seg, int strip,
 
     // the wave's boundary rows, if any: the special cases below are skipped in one test
     const bool edge = rw <= 0 || rw + R >= ny;
-    for (int it = 0; it < K; ++it) {
-        const bool bc = edge && it > 0;  // (the first iteration reads the boundary rows from memory)
-        ptp_barrier();
-        // V of the row below the wave's last one: column c at lane - 1
-        double nvx = vnext[-1], nvxp = vnext[0], nvyp = vnext[PTR_VROW];
-        const int rl = rw + R - 1;
-        if (bc && rl == ny - 1) {  // V row ny: Vx row ny = row ny-1, Vy zero
-            nvxp = vxp[R - 1];
-            nvx = lane_up(vxp[R - 1], 1);
-            nvyp = 0.0;
-        }
-        // V of the row of the wave's last row step (row 0: Vx row 0 = row 1, Vy row 0 zero)
-        double lvxp = vxp[R - 1], lvyp = vyp[R - 1];
-        if (bc && rl == 0) {
-            lvxp = nvxp;
-            lvyp = 0.0;
-        }
-        const double lvxc = lane_up(lvxp, 1), lvyc = lane_up(lvyp, 1);
-        const PTRCell last = ptr_cell(kc, lvxc, lvxp, lvyc, lvyp, nvx, nvxp, nvyp, m2[R - 1], mub[R - 1], taup[R - 1], pn[R - 1]);
-        cmine[0] = last.pn;
-        cmine[PTR_CROW] = last.txx;
-        cmine[2 * PTR_CROW] = last.txy;
-        cmine[3 * PTR_CROW] = last.tyy;
-        ptp_barrier();
-        PTRWin w;
-        w.pn = cprev[0];
-        w.dpn = (cprev[1] - w.pn) * kc.rdx;
-        w.dtxx = (cprev[PTR_CROW + 1] - cprev[PTR_CROW]) * kc.rdx;
-        w.txyp = cprev[2 * PTR_CROW + 1];
-        w.tyy = cprev[3 * PTR_CROW];
-        // V of the current row at columns c, c + 1
-        double cvxp = vxp[0], cvyp = vyp[0], cvx, cvy;
-        if (R == 1) {
-            cvxp = lvxp;
-            cvyp = lvyp;
-            cvx = lvxc;
-            cvy = lvyc;
-        } else {
-            if (bc && rw == 0) {
-                cvxp = vxp[R > 1 ? 1 : 0];
-                cvyp = 0.0;
-            }
-            cvx = lane_up(cvxp, 1);
-            cvy = lane_up(cvyp, 1);
-        }
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int r = rw + q;
-            double bvx, bvxp, bvy = 0.0, bvyp = 0.0;  // V of the row below
-            PTRCell s;
-            if (q == R - 1) {
-                bvx = nvx;
-                bvxp = nvxp;
-                s = last;
-            } else {
-                bvxp = vxp[q + 1 < R ? q + 1 : 0];
-                bvyp = vyp[q + 1 < R ? q + 1 : 0];
-                if (bc && r == ny - 1) {
-                    bvxp = cvxp;
-                    bvyp = 0.0;
-                }
-                if (bc && r + 1 == 0) {  // the row below is row 0
-                    bvxp = q + 2 < R ? vxp[q + 2 < R ? q + 2 : 0] : nvxp;
-                    bvyp = 0.0;
-                }
-                bvx = lane_up(bvxp, 1);
-                bvy = lane_up(bvyp, 1);
-                s = ptr_cell(kc, cvx, cvxp, cvy, cvyp, bvx, bvxp, bvyp, m2[q], mub[q], taup[q], pn[q]);
-            }
-            const double txyp = lane_down(s.txy, 1);
-            const double rx = (w.dtxx + (txyp - w.txyp) * kc.rdy) - w.dpn;
-            const double av4 = ((cvx + cvxp) + bvx) + bvxp;
-            const double ry = (((s.tyy - w.tyy) * kc.rdy + (txyp - s.txy) * kc.rdx) - (s.pn - w.pn) * kc.rdy) +
-                              kc.g * (rho1[q] - kc.dt * ((av4 * dxi[q]) * kc.rdx8 + (cvyp * dyi[q]) * kc.rdy2));
-            dvx[q] = kc.dampx * dvx[q] + rx;
-            dvy[q] = kc.dampy * dvy[q] + ry;
-            pn[q] = s.pn;
-            vxp[q] = cvxp + tauvx[q] * dvx[q];
-            vyp[q] = cvyp + tauvy[q] * dvy[q];
-            if (it < K - 1) ptp_bc(e, r == ny - 1, vxp[q], vyp[q]);
-            if (q < R - 1) {
-                w.dtxx = (lane_down(s.txx, 1) - s.txx) * kc.rdx;
-                w.dpn = (lane_down(s.pn, 1) - s.pn) * kc.rdx;
-                w.pn = s.pn;
-                w.tyy = s.tyy;
-                w.txyp = txyp;
-                cvx = bvx;
-                cvxp = bvxp;
-                cvy = bvy;
-                cvyp = bvyp;
-            }
-        }
-        vmine[0] = vxp[0];
-        vmine[PTR_VROW] = vyp[0];
-    }
     const bool out_lane = lane >= K && lane < SF_WAVE - K;
+    for (int pass = 0;; ++pass) {
+        const bool final_pass = !EX::RUN || pass == ex.passes - 1;
+        for (int it = 0; it < K; ++it) {
+            const bool bc = edge && (it > 0 || pass > 0);  // (the first iteration reads the boundary rows from memory)
+            ptp_barrier();
+            // V of the row below the wave's last one: column c at lane - 1
+            double nvx = vnext[-1], nvxp = vnext[0], nvyp = vnext[PTR_VROW];
+            const int rl = rw + R - 1;
+            if (bc && rl == ny - 1) {  // V row ny: Vx row ny = row ny-1, Vy zero
+                nvxp = vxp[R - 1];
+                nvx = lane_up(vxp[R - 1], 1);
+                nvyp = 0.0;
+            }
+            // V of the row of the wave's last row step (row 0: Vx row 0 = row 1, Vy row 0 zero)
+            double lvxp = vxp[R - 1], lvyp = vyp[R - 1];
+            if (bc && rl == 0) {
+                lvxp = nvxp;
+                lvyp = 0.0;
+            }
+            const double lvxc = lane_up(lvxp, 1), lvyc = lane_up(lvyp, 1);
+            const PTRCell last = ptr_cell(kc, lvxc, lvxp, lvyc, lvyp, nvx, nvxp, nvyp, m2[R - 1], mub[R - 1], taup[R - 1], pn[R - 1]);
+            cmine[0] = last.pn;
+            cmine[PTR_CROW] = last.txx;
+            cmine[2 * PTR_CROW] = last.txy;
+            cmine[3 * PTR_CROW] = last.tyy;
+            ptp_barrier();
+            PTRWin w;
+            w.pn = cprev[0];
+            w.dpn = (cprev[1] - w.pn) * kc.rdx;
+            w.dtxx = (cprev[PTR_CROW + 1] - cprev[PTR_CROW]) * kc.rdx;
+            w.txyp = cprev[2 * PTR_CROW + 1];
+            w.tyy = cprev[3 * PTR_CROW];
+            // V of the current row at columns c, c + 1
+            double cvxp = vxp[0], cvyp = vyp[0], cvx, cvy;
+            if (R == 1) {
+                cvxp = lvxp;
+                cvyp = lvyp;
+                cvx = lvxc;
+                cvy = lvyc;
+            } else {
+                if (bc && rw == 0) {
+                    cvxp = vxp[R > 1 ? 1 : 0];
+                    cvyp = 0.0;
+                }
+                cvx = lane_up(cvxp, 1);
+                cvy = lane_up(cvyp, 1);
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int r = rw + q;
+                double bvx, bvxp, bvy = 0.0, bvyp = 0.0;  // V of the row below
+                PTRCell s;
+                if (q == R - 1) {
+                    bvx = nvx;
+                    bvxp = nvxp;
+                    s = last;
+                } else {
+                    bvxp = vxp[q + 1 < R ? q + 1 : 0];
+                    bvyp = vyp[q + 1 < R ? q + 1 : 0];
+                    if (bc && r == ny - 1) {
+                        bvxp = cvxp;
+                        bvyp = 0.0;
+                    }
+                    if (bc && r + 1 == 0) {  // the row below is row 0
+                        bvxp = q + 2 < R ? vxp[q + 2 < R ? q + 2 : 0] : nvxp;
+                        bvyp = 0.0;
+                    }
+                    bvx = lane_up(bvxp, 1);
+                    bvy = lane_up(bvyp, 1);
+                    s = ptr_cell(kc, cvx, cvxp, cvy, cvyp, bvx, bvxp, bvyp, m2[q], mub[q], taup[q], pn[q]);
+                }
+                const double txyp = lane_down(s.txy, 1);
+                const double rx = (w.dtxx + (txyp - w.txyp) * kc.rdy) - w.dpn;
+                const double av4 = ((cvx + cvxp) + bvx) + bvxp;
+                const double ry = (((s.tyy - w.tyy) * kc.rdy + (txyp - s.txy) * kc.rdx) - (s.pn - w.pn) * kc.rdy) +
+                                  kc.g * (rho1[q] - kc.dt * ((av4 * dxi[q]) * kc.rdx8 + (cvyp * dyi[q]) * kc.rdy2));
+                dvx[q] = kc.dampx * dvx[q] + rx;
+                dvy[q] = kc.dampy * dvy[q] + ry;
+                pn[q] = s.pn;
+                vxp[q] = cvxp + tauvx[q] * dvx[q];
+                vyp[q] = cvyp + tauvy[q] * dvy[q];
+                if (it < K - 1 || !final_pass) ptp_bc(e, r == ny - 1, vxp[q], vyp[q]);
+                if (q < R - 1) {
+                    w.dtxx = (lane_down(s.txx, 1) - s.txx) * kc.rdx;
+                    w.dpn = (lane_down(s.pn, 1) - s.pn) * kc.rdx;
+                    w.pn = s.pn;
+                    w.tyy = s.tyy;
+                    w.txyp = txyp;
+                    cvx = bvx;
+                    cvxp = bvxp;
+                    cvy = bvy;
+                    cvyp = bvyp;
+                }
+            }
+            vmine[0] = vxp[0];
+            vmine[PTR_VROW] = vyp[0];
+        }
+        if (final_pass) break;
+        if constexpr (EX::RUN) {
+            const bool in_col = c >= 0 && c <= nx - 2, rim_lane = lane < 2 * K || lane >= SF_WAVE - 2 * K;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int r = rw + q;
+                if (r >= r0 && r < r1 && out_lane && in_col && (rim_lane || r < r0 + K || r >= r1 - K))
+                    ex.put(r, c, vxp[q], vyp[q], pn[q], dvx[q], dvy[q]);
+            }
+            if (!ex.swap()) return false;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int r = rw + q;
+                if (r >= 0 && r < ny && in_col && !(r >= r0 && r < r1 && out_lane))
+                    ex.get(r, c, vxp[q], vyp[q], pn[q], dvx[q], dvy[q]);
+            ptp_bc(e, r == ny - 1, vxp[q], vyp[q]);  // the boundary columns of the outer rows
+            }
+            vmine[0] = vxp[0];
+            vmine[PTR_VROW] = vyp[0];
+        }
+    }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
         const int r = rw + q;
@@ -250,6 +285,7 @@ __device__ __forceinline__ void ptr_tile(const PP& p, int K, int seg, int strip,
             pt2_store(p, o, c, r, r0, out_lane);
         }
     }
+    return true;
 }
 
 }  // namespace sf

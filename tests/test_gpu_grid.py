@@ -73,10 +73,10 @@ def test_grid_mode_more_tiles_than_waves(gpu):
     check_against_single(insts, outs, [G], iterMax=14)
 
 
-@pytest.mark.parametrize("nx,ny,cap", [(3, 3, 41), (40, 29, 333), (180, 700, 913), (700, 180, 1001), (930, 940, 40)])
+@pytest.mark.parametrize("nx,ny,cap", [(3, 3, 41), (40, 29, 333), (40, 200, 611), (180, 700, 913), (700, 180, 1001), (930, 940, 40)])
 def test_grid_mode_default_passes(gpu, nx, ny, cap):
-    """One, two and three rows per wave, passes cut short by checks, dt refreshes and the cap, and
-    several tiles per workgroup."""
+    """One, two and three rows per wave, tiles kept in registers with a reach of several segments,
+    passes cut short by checks, dt refreshes and the cap, and several tiles per workgroup."""
     S = cases.smooth_state(nx, ny, seed=630 + nx)
     insts = [(nx, ny, S, 1.0 / (nx - 1), 1.0 / (ny - 1))]
     pb, G = problem(S, nx, ny, insts[0][3], insts[0][4], iterMax=cap)
