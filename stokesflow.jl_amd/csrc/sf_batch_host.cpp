@@ -740,9 +740,13 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
         int64_t n32, n64, ncheck, ndtupdate, checked_at, window, left, wstart;
         double err_k, err_ref, dt_k, ws;
         bool converged;
+        // Between windows an instance waits for its new dt, then for its FP64 residual's sums.  The host
+        // reads either one step later, after the others' next pass is queued, so the GPU does not
+        // drain when a window ends.
+        enum { RUNS, WAITS_DT, WAITS_RESID } state;
     };
     res.assign((size_t)n, BatchResult{});
-    auto resid_err = [&](Run& r, double* err) -> int {
+    auto enqueue_resid = [&](Run& r) -> int {
         const sf_batch_instance& a = in[r.id];
         const RefineBufs& b = rb[(size_t)r.id];
         const SolveConsts k = solve_consts(a.nx, a.ny, a.dx, a.dy);
@@ -768,7 +772,14 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
         HIPCHK(launch_resid_f64(rp, nbr, s));
         double* h = env.hpart + (size_t)3 * RED_MAX_BLOCKS * r.id;
         HIPCHK(hipMemcpyAsync(h, b.part, 3 * (size_t)nbr * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
+        r.state = Run::WAITS_RESID;
+        return SF_OK;
+    };
+    auto resid_err = [&](const Run& r) -> double {  // once the copy has arrived
+        const sf_batch_instance& a = in[r.id];
+        const int64_t np = (int64_t)(a.nx - 1) * (a.ny - 1);
+        const int nbr = red_num_blocks(np);
+        const double* h = env.hpart + (size_t)3 * RED_MAX_BLOCKS * r.id;
         double sx = 0.0, sy = 0.0, sc = 0.0;
         for (int q = 0; q < nbr; ++q) {
             sx += h[q];
@@ -776,78 +787,67 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
             sc += h[2 * nbr + q];
         }
         const double n_rx = (double)(a.nx - 2) * (a.ny - 1), n_ry = (double)(a.nx - 1) * (a.ny - 2);
-        *err = std::max(std::max(sx / n_rx, sy / n_ry), sc / (double)np);
-        return SF_OK;
+        return std::max(std::max(sx / n_rx, sy / n_ry), sc / (double)np);
     };
-    // Runs checks / starts the next window; sets done when the instance has finished.
+    // With the residual's sums at hand: runs the check / starts the next window; sets done when the
+    // instance has finished.
     auto begin_window = [&](Run& r, bool* done) -> int {
         const sf_batch_instance& a = in[r.id];
         const BatchInstance& d = desc[(size_t)r.id];
         const RefineBufs& b = rb[(size_t)r.id];
         const int64_t nmx = (int64_t)(a.nx - 2) * (a.ny - 1), nmy = (int64_t)(a.nx - 1) * (a.ny - 2);
         *done = false;
-        for (;;) {
-            if (r.n32 >= a.iter_max) {
-                *done = true;
-                return SF_OK;
-            }
-            int rc = resid_err(r, &r.err_k);
-            if (rc) return rc;
-            if (!std::isfinite(r.err_k)) {
-                *done = true;
-                return SF_OK;
-            }
-            if (r.n32 > 0 && r.n32 % r.ncheck == 0 && r.n32 != r.checked_at && r.err_k <= a.eps) {
-                r.checked_at = r.n32;
-                float* const mxc = r.cur ? b.mx2 : b.mx;
-                float* const myc = r.cur ? b.my2 : b.my;
-                HIPCHK(launch_cast_f64(a.dVxdtau, mxc, nmx, s));
-                HIPCHK(launch_cast_f64(a.dVydtau, myc, nmy, s));
-                HIPCHK(launch_set_scalar(d.scal + SC_DT, r.dt_k, s));
-                rc = instance_check_iteration(s, a, d, b.part, env.w.hscal + (size_t)SC_COUNT * r.id, &r.err_ref);
-                if (rc) return rc;
-                r.n64 += 1;
-                HIPCHK(launch_cast_f32(mxc, a.dVxdtau, nmx, s));
-                HIPCHK(launch_cast_f32(myc, a.dVydtau, nmy, s));
-                if (r.err_ref <= a.eps) {
-                    r.converged = true;
-                    *done = true;
-                    return SF_OK;
-                }
-                continue;
-            }
-            const int64_t nvx = (int64_t)a.nx * (a.ny + 1), nvy = (int64_t)(a.nx + 1) * a.ny,
-                          np = (int64_t)(a.nx - 1) * (a.ny - 1);
-            for (int q = 0; q < 2; ++q) {
-                HIPCHK(launch_fill_f32(b.vx[q], nvx, 0.f, s));
-                HIPCHK(launch_fill_f32(b.vy[q], nvy, 0.f, s));
-                HIPCHK(launch_fill_f32(b.p[q], np, 0.f, s));
-            }
-            const float dtf = (float)r.dt_k;
-            if (cdesc[CDESC_PER_INST * (size_t)r.id].dt != dtf) {
-                for (int q = 0; q < CDESC_PER_INST; ++q) cdesc[CDESC_PER_INST * (size_t)r.id + q].dt = dtf;
-                env.hdt[r.id] = dtf;
-                for (int q = 0; q < CDESC_PER_INST; ++q)
-                    HIPCHK(hipMemcpyAsync((char*)(env.cdesc_dev + CDESC_PER_INST * (size_t)r.id + q) +
-                                              offsetof(CorrParams, dt),
-                                          env.hdt + r.id, sizeof(float), hipMemcpyHostToDevice, s));
-            }
-            int64_t steps = std::min(r.window, a.iter_max - r.n32);
-            steps = std::min(steps, r.ncheck - r.n32 % r.ncheck);
-            if (a.use_fss) steps = std::min(steps, r.ndtupdate - r.n32 % r.ndtupdate);
-            r.left = steps;
-            r.wstart = r.n32;
-            // both correction buffers are zero, so the window starts at the momentum's parity
+        r.err_k = resid_err(r);
+        if (!std::isfinite(r.err_k)) {
+            *done = true;
             return SF_OK;
         }
+        if (r.n32 > 0 && r.n32 % r.ncheck == 0 && r.n32 != r.checked_at && r.err_k <= a.eps) {
+            r.checked_at = r.n32;
+            float* const mxc = r.cur ? b.mx2 : b.mx;
+            float* const myc = r.cur ? b.my2 : b.my;
+            HIPCHK(launch_cast_f64(a.dVxdtau, mxc, nmx, s));
+            HIPCHK(launch_cast_f64(a.dVydtau, myc, nmy, s));
+            HIPCHK(launch_set_scalar(d.scal + SC_DT, r.dt_k, s));
+            const int rc = instance_check_iteration(s, a, d, b.part, env.w.hscal + (size_t)SC_COUNT * r.id, &r.err_ref);
+            if (rc) return rc;
+            r.n64 += 1;
+            HIPCHK(launch_cast_f32(mxc, a.dVxdtau, nmx, s));
+            HIPCHK(launch_cast_f32(myc, a.dVydtau, nmy, s));
+            if (r.err_ref <= a.eps) {
+                r.converged = true;
+                *done = true;
+                return SF_OK;
+            }
+            return enqueue_resid(r);  // of the state after the check's iteration
+        }
+        const int64_t nvx = (int64_t)a.nx * (a.ny + 1), nvy = (int64_t)(a.nx + 1) * a.ny,
+                      np = (int64_t)(a.nx - 1) * (a.ny - 1);
+        HIPCHK(launch_fill_f32(b.vx[0], 2 * (nvx + nvy + np), 0.f, s));  // both corrections (refine_carve)
+        const float dtf = (float)r.dt_k;
+        if (cdesc[CDESC_PER_INST * (size_t)r.id].dt != dtf) {
+            for (int q = 0; q < CDESC_PER_INST; ++q) cdesc[CDESC_PER_INST * (size_t)r.id + q].dt = dtf;
+            env.hdt[r.id] = dtf;
+            for (int q = 0; q < CDESC_PER_INST; ++q)
+                HIPCHK(hipMemcpyAsync((char*)(env.cdesc_dev + CDESC_PER_INST * (size_t)r.id + q) +
+                                          offsetof(CorrParams, dt),
+                                      env.hdt + r.id, sizeof(float), hipMemcpyHostToDevice, s));
+        }
+        int64_t steps = std::min(r.window, a.iter_max - r.n32);
+        steps = std::min(steps, r.ncheck - r.n32 % r.ncheck);
+        if (a.use_fss) steps = std::min(steps, r.ndtupdate - r.n32 % r.ndtupdate);
+        r.left = steps;
+        r.wstart = r.n32;
+        r.state = Run::RUNS;
+        // both correction buffers are zero, so the window starts at the momentum's parity
+        return SF_OK;
     };
     auto end_window = [&](Run& r) -> int {
         const sf_batch_instance& a = in[r.id];
         const BatchInstance& d = desc[(size_t)r.id];
         const RefineBufs& b = rb[(size_t)r.id];
-        HIPCHK(launch_update_f64(a.Vx_s, b.vx[r.cur], (int64_t)a.nx * (a.ny + 1), s));
-        HIPCHK(launch_update_f64(a.Vy_s, b.vy[r.cur], (int64_t)(a.nx + 1) * a.ny, s));
-        HIPCHK(launch_update_f64(a.P, b.p[r.cur], (int64_t)(a.nx - 1) * (a.ny - 1), s));
+        HIPCHK(launch_update_state(a.Vx_s, b.vx[r.cur], (int64_t)a.nx * (a.ny + 1), a.Vy_s, b.vy[r.cur],
+                                   (int64_t)(a.nx + 1) * a.ny, a.P, b.p[r.cur], (int64_t)(a.nx - 1) * (a.ny - 1), s));
         r.rebases += 1;
         // the reference refreshes the stabilisation dt every ndtupdate iterations (:60-62)
         if (a.use_fss && (r.n32 / r.ndtupdate) > (r.wstart / r.ndtupdate)) {
@@ -855,10 +855,10 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
             if (rc) return rc;
             double* hs = env.w.hscal + (size_t)SC_COUNT * r.id;
             HIPCHK(hipMemcpyAsync(hs, d.scal, SC_COUNT * sizeof(double), hipMemcpyDeviceToHost, s));
-            HIPCHK(hipStreamSynchronize(s));
-            r.dt_k = hs[SC_DT_CHECK];
+            r.state = Run::WAITS_DT;
+            return SF_OK;
         }
-        return SF_OK;
+        return r.n32 < a.iter_max ? enqueue_resid(r) : SF_OK;  // (an instance at its cap needs none)
     };
     auto finish = [&](const Run& r) -> int {
         const sf_batch_instance& a = in[r.id];
@@ -888,6 +888,14 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
     wa.desc = env.cdesc_dev;
     CorrPlan plan{};
     bool replan = true;  // the active set has changed
+    struct Event {
+        hipEvent_t e = nullptr;
+        ~Event()
+        {
+            if (e) (void)hipEventDestroy(e);
+        }
+    } ev;
+    HIPCHK(hipEventCreateWithFlags(&ev.e, hipEventDisableTiming));
     int rc = SF_OK;
     while (!act.empty() || q < order.size()) {
         while (q < order.size() && (int)act.size() < WIDE_MAX &&
@@ -910,17 +918,16 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
             HIPCHK(launch_cast_f32(b.mup, a.mu_p, (int64_t)(a.nx - 1) * (a.ny - 1), s));
             HIPCHK(launch_cast_f32(b.mx, a.dVxdtau, (int64_t)(a.nx - 2) * (a.ny - 1), s));
             HIPCHK(launch_cast_f32(b.my, a.dVydtau, (int64_t)(a.nx - 1) * (a.ny - 2), s));
-            bool done = false;
-            rc = begin_window(r, &done);
-            if (rc) return rc;
-            if (done) {
+            if (a.iter_max < 1) {
                 rc = finish(r);
                 if (rc) return rc;
-            } else {
-                act.push_back(r);
-                ws_active += r.ws;
-                replan = true;
+                continue;
             }
+            rc = enqueue_resid(r);
+            if (rc) return rc;
+            act.push_back(r);
+            ws_active += r.ws;
+            replan = true;
         }
         if (act.empty()) continue;
         if (replan) {
@@ -933,32 +940,46 @@ int batch_run_wide_refined(const RefineEnv& env, const sf_batch_instance* in, in
             for (size_t j = 0; j < act.size(); ++j) act[j].kmax = k[j];
             replan = false;
         }
-        // one launch: every instance as many sweeps as its plan has and its window leaves
+        // what an instance waits for was queued before this step's pass: marked here, read after the pass
+        const bool waiting = std::any_of(act.begin(), act.end(), [](const Run& r) { return r.state != Run::RUNS; });
+        if (waiting) HIPCHK(hipEventRecord(ev.e, s));
+        // one launch: every running instance as many sweeps as its plan has and its window leaves
         int tiles = 0;
-        for (size_t j = 0; j < act.size(); ++j) {
-            Run& r = act[j];
+        wa.n_active = 0;
+        for (Run& r : act) {
+            if (r.state != Run::RUNS) continue;
+            const int j = wa.n_active++;
             r.k = (int)std::min<int64_t>(r.kmax, r.left);
             wa.tile_start[j] = tiles;
             wa.slot_desc[j] = CDESC_PER_INST * r.id + r.cur;
             wa.slot_k[j] = r.k;
             tiles += corr_plan_tiles(plan, in[r.id].nx, in[r.id].ny, r.k);
         }
-        wa.n_active = (int)act.size();
         wa.tile_start[wa.n_active] = tiles;
-        HIPCHK(launch_wide_corr(wa, plan, s));
+        if (wa.n_active) HIPCHK(launch_wide_corr(wa, plan, s));
+        if (wa.n_active == 0) HIPCHK(hipStreamSynchronize(s));
+        else if (waiting) HIPCHK(hipEventSynchronize(ev.e));
         std::vector<Run> keep;
         keep.reserve(act.size());
         for (Run& r : act) {
-            r.cur ^= 1;
-            r.n32 += r.k;
-            r.left -= r.k;
+            const sf_batch_instance& a = in[r.id];
             bool done = false;
-            if (r.left == 0) {
-                rc = end_window(r);
-                if (rc) return rc;
+            if (r.state == Run::RUNS) {
+                r.cur ^= 1;
+                r.n32 += r.k;
+                r.left -= r.k;
+                if (r.left == 0) {
+                    rc = end_window(r);
+                    done = r.state == Run::RUNS;  // at its cap
+                }
+            } else if (r.state == Run::WAITS_DT) {
+                r.dt_k = env.w.hscal[(size_t)SC_COUNT * r.id + SC_DT_CHECK];
+                if (r.n32 >= a.iter_max) done = true;
+                else rc = enqueue_resid(r);
+            } else {
                 rc = begin_window(r, &done);
-                if (rc) return rc;
             }
+            if (rc) return rc;
             if (done) {
                 rc = finish(r);
                 if (rc) return rc;

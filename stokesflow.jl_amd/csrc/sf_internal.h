@@ -177,6 +177,8 @@ CorrPlan corr_plan(const int* nx, const int* ny, int n, int* k);
 int corr_plan_tiles(const CorrPlan& plan, int nx, int ny, int k);
 hipError_t launch_resid_f64(const ResidParams& p, int nb, hipStream_t s);
 hipError_t launch_update_f64(double* a, const float* d, int64_t n, hipStream_t s);
+hipError_t launch_update_state(double* a, const float* da, int64_t na, double* b, const float* db, int64_t nb, double* c,
+                               const float* dc, int64_t nc, hipStream_t s);
 hipError_t launch_cast_f32(float* dst, const double* src, int64_t n, hipStream_t s);
 hipError_t launch_fill_f32(float* dst, int64_t n, float v, hipStream_t s);
 hipError_t launch_fill_f64(double* dst, int64_t n, double v, hipStream_t s);

@@ -796,6 +796,26 @@ hipError_t launch_update_f64(double* a, const float* d, int64_t n, hipStream_t s
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void update_state_f64(double* a, const float* da, int64_t na, double* b, const float* db,
+                                                       int64_t nb, double* c, const float* dc, int64_t nc)
+{
+    double* const u = blockIdx.y == 0 ? a : blockIdx.y == 1 ? b : c;
+    const float* const d = blockIdx.y == 0 ? da : blockIdx.y == 1 ? db : dc;
+    const int64_t n = blockIdx.y == 0 ? na : blockIdx.y == 1 ? nb : nc;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
+        u[k] = u[k] + (double)d[k];
+}
+
+// The three fields of the state in one launch.
+hipError_t launch_update_state(double* a, const float* da, int64_t na, double* b, const float* db, int64_t nb, double* c,
+                               const float* dc, int64_t nc, hipStream_t s)
+{
+    const int64_t n = std::max(na, std::max(nb, nc));
+    const int blocks = (int)std::min<int64_t>((n + 255) / 256, 2048);
+    hipLaunchKernelGGL(update_state_f64, dim3(blocks, 3), dim3(256), 0, s, a, da, na, b, db, nb, c, dc, nc);
+    return hipGetLastError();
+}
+
 hipError_t launch_cast_f32(float* dst, const double* src, int64_t n, hipStream_t s)
 {
     hipLaunchKernelGGL(cast_f32, dim3(grid_for(n)), dim3(256), 0, s, dst, src, n);
