@@ -701,9 +701,9 @@ def main():
         if c32:
             k32 = c32["iters_per_launch"]
             b32 = bytes_per_iter_fp32(nx, ny)
-            kname = f"pt_corrk_f32<{k32}>" if k32 >= 3 else {1: "pt_corr_f32", 2: "pt_corr2_f32"}[k32]
+            kname = f"ctr_tile_f32, {k32} sweeps"  # the size default's pass
             line["roofline_fp32"] = roofline_entry(kname, k32, c32["launch_s"], c32["launches"], b32, b32,
-                                                   profiled_traffic(nx, f"pt_corrk{k32}_f32"), probe)
+                                                   profiled_traffic(nx, f"ctr{k32}_tile_f32"), probe)
             line["refined_sweeps"]["kernel_s_per_sweep"] = c32["launch_s"] / k32
     note("cpu baseline and refined passes done")
     if not a.no_ref_window:

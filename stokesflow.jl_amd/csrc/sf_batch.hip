@@ -308,6 +308,134 @@ hipError_t launch_wide_pt2(const WideArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------------------
+// Wide mode: the dt refreshes and checks of all instances of a step in four launches (one instance at a
+// time took seven launches and a copy each: half the time of 64 instances of 64^2).  Every instance's
+// sums have the single solver's blocks and order, so its err has the same bits.
+
+// |Vx|, |Vy| maxima per block, as reduce_abs_partials.
+__global__ __launch_bounds__(256) void wide_dt_partials(WideCheckArgs a)
+{
+    __shared__ double sh[256];
+    const int z = blockIdx.z, nb = a.nb_dt[z], t = threadIdx.x;
+    if ((int)blockIdx.x >= nb) return;
+    CBatch& I = ((CBatch*)a.desc)[a.slot_inst[z]];
+    const PTParams SF_CONST& p = I.wpt[a.slot_pf[z] & 1];
+    const double* __restrict__ src = blockIdx.y ? p.vy_b : p.vx_b;
+    const int64_t n = blockIdx.y ? (int64_t)(I.nx + 1) * I.ny : (int64_t)I.nx * (I.ny + 1);
+    double acc = -__builtin_inf();
+    for (int64_t k = (int64_t)blockIdx.x * 256 + t; k < n; k += (int64_t)nb * 256) acc = jl_max(acc, fabs(src[k]));
+    sh[t] = acc;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (t < s) sh[t] = jl_max(sh[t], sh[t + s]);
+        __syncthreads();
+    }
+    if (t == 0) a.part[(int64_t)z * 3 * RED_MAX_BLOCKS + (int64_t)blockIdx.y * nb + blockIdx.x] = sh[0];
+}
+
+// dt = maxdisp * min(dx / max|Vx|, dy / max|Vy|) (compute_dt, :118-121); 0 without stabilisation.
+__global__ __launch_bounds__(64) void wide_dt_final(WideCheckArgs a)
+{
+    const int z = blockIdx.x, nb = a.nb_dt[z], lane = threadIdx.x;
+    CBatch& I = ((CBatch*)a.desc)[a.slot_inst[z]];
+    const double* part = a.part + (int64_t)z * 3 * RED_MAX_BLOCKS;
+    double mx = -__builtin_inf(), my = -__builtin_inf();
+    for (int b = lane; b < nb; b += 64) {
+        mx = jl_max(mx, part[b]);
+        my = jl_max(my, part[nb + b]);
+    }
+    for (int d = 32; d >= 1; d >>= 1) {
+        mx = jl_max(mx, __shfl_xor(mx, d, 64));
+        my = jl_max(my, __shfl_xor(my, d, 64));
+    }
+    if (lane != 0) return;
+    const double dtc = nb ? I.maxdisp * jl_min(I.dx / mx, I.dy / my) : 0.0;
+    I.scal[SC_DT_CHECK] = dtc;
+    if (a.slot_pf[z] & WIDE_CHECK_DT) I.scal[SC_DT] = dtc;
+}
+
+// Sums of |Rx|, |Ry| and |divV| per block; Ry (compute_Residuals!, :189-202, post-update V and dt_check) is
+// formed on the way.
+__global__ __launch_bounds__(256) void wide_err_partials(WideCheckArgs a)
+{
+    __shared__ double sh[256];
+    const int z = blockIdx.z, nb = a.nb_err[z], t = threadIdx.x;
+    if ((int)blockIdx.x >= nb) return;
+    CBatch& I = ((CBatch*)a.desc)[a.slot_inst[z]];
+    const PTParams SF_CONST& p = I.wpt[a.slot_pf[z] & 1];
+    const int nx = I.nx, ny = I.ny;
+    double acc = 0.0;
+    if (blockIdx.y == 1) {
+        const int64_t n = (int64_t)(nx - 1) * (ny - 2), lp = nx - 1, lvx = nx, lvy = nx + 1, lr = nx + 1;
+        const double dt = I.scal[SC_DT_CHECK], rdx = p.rdx, rdy = p.rdy, g = p.g;
+        const double* __restrict__ vx = p.vx_b;
+        const double* __restrict__ vy = p.vy_b;
+        const double* __restrict__ P = p.p_b;
+        const double* __restrict__ rho = p.rho;
+        const double* __restrict__ tyy = p.tyy;
+        const double* __restrict__ txy = p.txy;
+        for (int64_t k = (int64_t)blockIdx.x * 256 + t; k < n; k += (int64_t)nb * 256) {
+            const int i = (int)(k % (nx - 1)), j = (int)(k / (nx - 1));
+            const double av = 0.25 * (((vx[ix2(i, j + 1, lvx)] + vx[ix2(i + 1, j + 1, lvx)]) + vx[ix2(i, j + 2, lvx)]) +
+                                      vx[ix2(i + 1, j + 2, lvx)]);
+            const double d_xi = rho[ix2(i + 2, j + 1, lr)] - rho[ix2(i, j + 1, lr)];
+            const double d_yi = rho[ix2(i + 1, j + 2, lr)] - rho[ix2(i + 1, j, lr)];
+            const double ry =
+                (((tyy[ix2(i, j + 1, lp)] - tyy[ix2(i, j, lp)]) * rdy + (txy[ix2(i + 1, j + 1, lvx)] - txy[ix2(i, j + 1, lvx)]) * rdx) -
+                 (P[ix2(i, j + 1, lp)] - P[ix2(i, j, lp)]) * rdy) +
+                g * (rho[ix2(i + 1, j + 1, lr)] - dt * (((av * d_xi) * 0.5) * rdx + ((vy[ix2(i + 1, j + 1, lvy)] * d_yi) * 0.5) * rdy));
+            acc = acc + fabs(ry);
+        }
+    } else {
+        const double* __restrict__ src = blockIdx.y ? p.divv : p.rx;
+        const int64_t n = blockIdx.y ? (int64_t)(nx - 1) * (ny - 1) : (int64_t)(nx - 2) * (ny - 1);
+        for (int64_t k = (int64_t)blockIdx.x * 256 + t; k < n; k += (int64_t)nb * 256) acc = acc + fabs(src[k]);
+    }
+    sh[t] = acc;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (t < s) sh[t] = sh[t] + sh[t + s];
+        __syncthreads();
+    }
+    if (t == 0) a.part[(int64_t)z * 3 * RED_MAX_BLOCKS + (int64_t)blockIdx.y * nb + blockIdx.x] = sh[0];
+}
+
+// err = max(mean|Rx|, mean|Ry|, mean|divV|) (compute_err, :103-109), lane a summing array a's blocks in order,
+// and the instance's scalars into pinned host memory.
+__global__ __launch_bounds__(64) void wide_err_final(WideCheckArgs a)
+{
+    const int z = blockIdx.x, nb = a.nb_err[z], lane = threadIdx.x;
+    if (nb == 0) return;
+    CBatch& I = ((CBatch*)a.desc)[a.slot_inst[z]];
+    const double* part = a.part + (int64_t)z * 3 * RED_MAX_BLOCKS + (int64_t)min(lane, 2) * nb;
+    double s = 0.0;
+    for (int b = 0; b < nb; ++b) s = s + part[b];
+    const double s0 = __shfl(s, 0), s1 = __shfl(s, 1), s2 = __shfl(s, 2);
+    if (lane != 0) return;
+    const double n_rx = (double)(I.nx - 2) * (I.ny - 1), n_ry = (double)(I.nx - 1) * (I.ny - 2),
+                 n_dv = (double)(I.nx - 1) * (I.ny - 1);
+    I.scal[SC_ERR] = jl_max(jl_max(s0 / n_rx, s1 / n_ry), s2 / n_dv);
+    for (int q = 0; q < SC_COUNT; ++q) a.hscal[(int64_t)SC_COUNT * a.slot_inst[z] + q] = I.scal[q];
+}
+
+hipError_t launch_wide_check(const WideCheckArgs& a, hipStream_t s)
+{
+    int dt = 0, err = 0;
+    for (int z = 0; z < a.n; ++z) {
+        dt = std::max(dt, a.nb_dt[z]);
+        err = std::max(err, a.nb_err[z]);
+    }
+    if (a.n <= 0) return hipSuccess;
+    if (dt) hipLaunchKernelGGL(wide_dt_partials, dim3(dt, 2, a.n), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(wide_dt_final, dim3(a.n), dim3(64), 0, s, a);
+    if (err) {
+        hipLaunchKernelGGL(wide_err_partials, dim3(err, 3, a.n), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(wide_err_final, dim3(a.n), dim3(64), 0, s, a);
+    }
+    return hipGetLastError();
+}
+
 __global__ void zero_int(int* p) { *p = 0; }
 
 int batch_blocks_per_cu(int threads)

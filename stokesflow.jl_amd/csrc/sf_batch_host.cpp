@@ -333,6 +333,11 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
     bool step_checked[2] = {false, false};
     int64_t step = 0;
     WideArgs wa, w2, w3, w4, wr, wp;
+    WideCheckArgs wc;
+    std::memset(&wc, 0, sizeof(wc));
+    wc.desc = env.desc_dev;
+    wc.part = env.part;
+    wc.hscal = env.hscal;
     WidePlan plan{};      // of the resident passes, for the active instances without a tuned shape
     bool replan = true;   // the active set has changed
     std::memset(&wa, 0, sizeof(wa));
@@ -457,60 +462,21 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
         if (w2.n_active) HIPCHK(launch_wide_pt2(w2, s));
         if (wa.n_active) HIPCHK(launch_wide_pt(wa, depth, s));
         bool any_check = false;
+        wc.n = 0;
         for (Run& r : act) {
             if (r.skip) continue;
             const sf_batch_instance& a = in[r.id];
-            const BatchInstance& d = desc[(size_t)r.id];
-            const PTParams& p = d.wpt[r.nlaunch & 1];  // its outputs are now the current state
             const int64_t it_done = r.iter + r.k - 1;  // the last iteration just run
             const bool dt_upd = a.use_fss && (it_done % r.ndtupdate) == 0;
-            if (dt_upd) {
-                rc = enqueue_dt_raw(s, a.nx, a.ny, p.vx_b, p.vy_b, a.dx, a.dy, a.maxdisp, 1, env.part, d.scal);
-                if (rc) return rc;
-            }
-            if (!r.checking) continue;
-            any_check = true;
-            if (a.use_fss) {
-                if (!dt_upd) {
-                    rc = enqueue_dt_raw(s, a.nx, a.ny, p.vx_b, p.vy_b, a.dx, a.dy, a.maxdisp, 0, env.part, d.scal);
-                    if (rc) return rc;
-                }
-            } else {
-                HIPCHK(launch_set_scalar(d.scal + SC_DT_CHECK, 0.0, s));
-            }
-            const SolveConsts k = solve_consts(a.nx, a.ny, a.dx, a.dy);
-            ResYParams rq{};
-            rq.nx = a.nx;
-            rq.ny = a.ny;
-            rq.tyy = p.tyy;
-            rq.txy = p.txy;
-            rq.P = p.p_b;
-            rq.rho = a.rho_vy;
-            rq.vx = p.vx_b;
-            rq.vy = p.vy_b;
-            rq.dt = d.scal + SC_DT_CHECK;
-            rq.ry = d.ry;
-            rq.g = a.g_y;
-            rq.rdx = k.rdx;
-            rq.rdy = k.rdy;
-            HIPCHK(launch_pt_resid_y(rq, s));
-            const double n_rx = (double)(a.nx - 2) * (a.ny - 1), n_ry = (double)(a.nx - 1) * (a.ny - 2),
-                         n_dv = (double)(a.nx - 1) * (a.ny - 1);
-            RedParams rp{};
-            rp.a[0] = p.rx;
-            rp.n[0] = (int64_t)n_rx;
-            rp.a[1] = d.ry;
-            rp.n[1] = (int64_t)n_ry;
-            rp.a[2] = p.divv;
-            rp.n[2] = (int64_t)n_dv;
-            rp.part = env.part;
-            rp.mode = RED_SUM;
-            const int nb = red_num_blocks((int64_t)n_dv);
-            HIPCHK(launch_reduce(rp, 3, nb, s));
-            HIPCHK(launch_finalize_err(env.part, nb, n_rx, n_ry, n_dv, d.scal, s));
-            HIPCHK(hipMemcpyAsync(env.hscal + (size_t)SC_COUNT * r.id, d.scal, SC_COUNT * sizeof(double),
-                                  hipMemcpyDeviceToHost, s));
+            if (!dt_upd && !r.checking) continue;
+            const int z = wc.n++;
+            wc.slot_inst[z] = r.id;
+            wc.slot_pf[z] = (int)(r.nlaunch & 1) | (dt_upd ? WIDE_CHECK_DT : 0);  // that pass's outputs are the state
+            wc.nb_dt[z] = a.use_fss ? red_num_blocks(std::max((int64_t)a.nx * (a.ny + 1), (int64_t)(a.nx + 1) * a.ny)) : 0;
+            wc.nb_err[z] = r.checking ? red_num_blocks((int64_t)(a.nx - 1) * (a.ny - 1)) : 0;
+            any_check = any_check || r.checking;
         }
+        HIPCHK(launch_wide_check(wc, s));
         const int sp = (int)(step & 1);
         step_checked[sp] = any_check;
         if (any_check) HIPCHK(hipEventRecord(ev.e[sp], s));
@@ -1127,7 +1093,8 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         // 15.38 at 1536 and 3072 MiB (64 slots full of 512^2 instances: 18,432 waves, nine full rounds of
         // the 2,048 resident ones); 128 slots were slower (15.5 s)
         const double budget = (prm && prm->budget_mb > 0.0) ? prm->budget_mb * 1048576.0 : 1536.0 * 1048576.0;
-        const WideEnv env{s, c->b_inst, c->part, c->b_hscal};
+        if (!c->b_wpart) HIPCHK(dalloc(&c->b_wpart, (size_t)3 * RED_MAX_BLOCKS * WIDE_MAX));
+        const WideEnv env{s, c->b_inst, c->b_wpart, c->b_hscal};
         rc = batch_run_wide(env, in, n, host, order, budget, (prm && prm->depth > 1) ? 2 : 1, res);
         if (rc) return rc;
     } else {

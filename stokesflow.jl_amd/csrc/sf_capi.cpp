@@ -38,7 +38,7 @@ static void free_ctx(sf_ctx* c)
         if (b) (void)hipFree(b);
     if (c->hpart) (void)hipHostFree(c->hpart);
     if (c->b_hscal) (void)hipHostFree(c->b_hscal);
-    for (void* b : {(void*)c->b_pool32, (void*)c->b_part, (void*)c->b_cdesc})
+    for (void* b : {(void*)c->b_pool32, (void*)c->b_part, (void*)c->b_wpart, (void*)c->b_cdesc})
         if (b) (void)hipFree(b);
     for (void* b : {(void*)c->b_hpart, (void*)c->b_hdt})
         if (b) (void)hipHostFree(b);

@@ -231,7 +231,7 @@ extern "C" int sf_ensemble_create(sf_ctx* c, const sf_step_args* members, int n,
     if (er == hipSuccess) er = dalloc(&e->queue, 1);
     if (er == hipSuccess) er = dalloc(&e->res, (size_t)n);
     if (er == hipSuccess) er = dalloc(&e->cnt, (size_t)ENS_CNT * n);
-    if (er == hipSuccess) er = dalloc(&e->part, 3 * (size_t)RED_MAX_BLOCKS);
+    if (er == hipSuccess) er = dalloc(&e->part, 3 * (size_t)RED_MAX_BLOCKS * WIDE_MAX);
     if (er == hipSuccess) er = hipHostMalloc((void**)&e->hcnt, sizeof(unsigned long long) * ENS_CNT * n, hipHostMallocDefault);
     if (er == hipSuccess) er = hipHostMalloc((void**)&e->hres, sizeof(BatchResult) * n, hipHostMallocDefault);
     if (er == hipSuccess) er = hipHostMalloc((void**)&e->hscal, sizeof(double) * SC_COUNT * n, hipHostMallocDefault);

@@ -47,7 +47,7 @@ int m2g_reserve(M2GScratch& S, int64_t nm, int64_t ncells);
 // err back, as the reference does), retires converged instances and refills the set from the
 // largest-first queue.  Every instance runs exactly the iterations of solveStokes!.
 // Buffers a wide-mode run uses: its stream, device descriptors, reduction partials
-// (3 * RED_MAX_BLOCKS) and pinned per-instance scalars (SC_COUNT per instance).
+// (FP64: 3 * RED_MAX_BLOCKS per active instance) and pinned per-instance scalars (SC_COUNT per instance).
 struct WideEnv {
     hipStream_t s;
     const BatchInstance* desc_dev;
@@ -255,6 +255,7 @@ struct sf_ctx {
     float* b_pool32 = nullptr;
     size_t b_pool32_cap = 0;
     double* b_part = nullptr;      // 3 * RED_MAX_BLOCKS per instance
+    double* b_wpart = nullptr;     // wide FP64 mode: 3 * RED_MAX_BLOCKS per active instance
     sf::CorrParams* b_cdesc = nullptr;  // CDESC_PER_INST per instance
     double* b_hpart = nullptr;     // pinned
     float* b_hdt = nullptr;        // pinned

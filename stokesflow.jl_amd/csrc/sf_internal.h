@@ -292,6 +292,20 @@ WidePlan wide_plan(const int* nx, const int* ny, int n, int* k, int* rows);
 int wide_resident_tiles(const WidePlan& plan, int nx, int ny, int k);
 hipError_t launch_wide_resident(const WideArgs& a, const WidePlan& plan, hipStream_t s);
 
+// Wide mode: dt refreshes and checks of slot i = 0..n-1 (instance slot_inst[i], outputs of the pass of parity
+// slot_pf[i] & 1).  nb_dt: blocks of the velocity maxima (0: dt_check = 0), nb_err: of the check's sums (0: no
+// check); WIDE_CHECK_DT: the new dt is the stabilisation's, too.  part: 3 * RED_MAX_BLOCKS per slot; hscal:
+// pinned, SC_COUNT per instance, written where there is a check.
+#define WIDE_CHECK_DT 2
+struct WideCheckArgs {
+    const BatchInstance* desc;
+    int n;
+    int slot_inst[WIDE_MAX], slot_pf[WIDE_MAX], nb_dt[WIDE_MAX], nb_err[WIDE_MAX];
+    double* part;
+    double* hscal;
+};
+hipError_t launch_wide_check(const WideCheckArgs& a, hipStream_t s);
+
 // Wide mode of the FP32 correction sweeps: slot i runs slot_k[i] sweeps on descriptor slot_desc[i] (two
 // descriptors per instance, one per ping-pong direction).
 struct WideCorrArgs {
