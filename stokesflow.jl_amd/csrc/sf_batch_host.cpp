@@ -14,8 +14,8 @@ namespace sf {
 // The same where every tile stays in registers: the exchange with the tiles around (600x520 takes 2.30 us
 // per iteration planned with 3.5, 2.65 with 4.5; 64^2 1.34 with both, 1.46 with 6).
 #define GRID_KEPT_US 3.5
-// The grids that resident passes are for (us per iteration, and with one-wave passes of three): 64^2 1.34,
-// 3.48; 301x257 1.56, 4.09; 384x300 1.62, 6.49; 512^2 2.13, 8.04; 730^2 4.0, 10.6; past what the chip holds
+// The grids that resident passes are for (us per iteration, and with one-wave passes of three): 64^2 1.27,
+// 3.48; 301x257 1.53, 4.09; 384x300 1.58, 6.49; 512^2 2.11, 8.04; 730^2 4.1, 10.6; past what the chip holds
 // at once 1000x777 8.3, 9.6; 1024^2 11.3, 10.9, and larger ones the same within 7%.
 #define GRID_RESIDENT_NODES 900000
 

@@ -7,7 +7,7 @@
 // separates the passes.  Small and middle grids take passes of up to GRID_RESIDENT_MAX_K iterations on
 // tiles in registers, a tile per workgroup of up to 16 waves.  Where the chip holds all tiles at once they
 // stay there from pass to pass, and only the nodes that other tiles need go through memory, each tile
-// waiting for its neighbours alone (GridExchange: 384x300 takes 1.62 us per iteration; 2.46 where every
+// waiting for its neighbours alone (GridExchange: 384x300 takes 1.58 us per iteration; 2.46 where every
 // pass met at the barrier and read its tile again, which costs 8 us, and 6.5 with passes of three).
 // Larger grids take passes of up to three on
 // tiles of one wave, one to eight waves per workgroup.  Tiles go out t = band, band + G, ... (the
@@ -260,8 +260,21 @@ struct GridExchange {
                 __hip_atomic_store(flags + 16 * (segid * nstrips + strip), seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const int ds = (int)threadIdx.x % 3 - 1, dg = (int)threadIdx.x / 3 - reach;
             const int ns = strip + ds, ng = segid + dg;
-            if (dg <= reach && ns >= 0 && ns < nstrips && ng >= 0 && ng < nseg)
-                ok = wait_agent(flags + 16 * (ng * nstrips + ns), seq, s, limit);
+            const bool mine = dg <= reach && ns >= 0 && ns < nstrips && ng >= 0 && ng < nseg;
+            const u64* const flag = flags + (mine ? 16 * (ng * nstrips + ns) : 16 * (segid * nstrips + strip));
+            // as wait_agent, for all neighbours at once, the failure flag read along with theirs
+            const uint64_t t0 = wall_clock64();
+            while (true) {
+                const u64 have = ld_agent(flag), failed = ld_agent(s + GRID_SYNC_FAIL);
+                if (!__ballot(have < seq)) break;
+                if (failed != 0ull) ok = 0;
+                if (wall_clock64() - t0 > limit) {
+                    __hip_atomic_store(s + GRID_SYNC_FAIL, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(s + GRID_SYNC_STICKY, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    ok = 0;
+                }
+                if (__ballot(!ok)) break;
+            }
         }
         return __syncthreads_or(!ok) == 0;
     }
