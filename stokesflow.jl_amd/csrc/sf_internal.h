@@ -331,7 +331,7 @@ struct M2GScratch {
     int64_t cap_markers = 0;
     int64_t cap_cells = 0;
     int* key = nullptr;      // [nm] cell key or -1
-    int* loc = nullptr;      // [nm] place in the cell; after the scatter, two lists of tiles and parts
+    int* loc = nullptr;      // [nm] place in the cell; after the scatter, two lists of parts of tiles and of rows
     int* count = nullptr;    // [cells]
     int* offset = nullptr;   // [cells + 1]
     int* rec_idx = nullptr;  // [nm] marker index in cell order

@@ -17,8 +17,8 @@
 //               cell's markers by index, and merges the four cells of each node by index: that
 //               replays exactly the CPU accumulation order, so wt_sum and val_wt_sum are the CPU
 //               sums; safeDivision (:164-172) keeps the old value where wt == 0.
-//   5. tiles whose markers do not fit into LDS are done in parts; parts that do not fit either, and all
-//               of a grid with very many markers per cell, from global memory, a wave per node.
+//   5. tiles whose markers do not fit into LDS are done in pieces of fewer rows; rows that do not fit alone,
+//               and all of a grid with very many markers per cell, from global memory, a wave per node.
 #include <algorithm>
 
 #include "sf_device.h"
@@ -240,12 +240,12 @@ struct M2GNodes {
     double xmin, ymin, dx, dy;
     int gnx, gny;
     int tx, ty, ntx, nty;  // nodes per tile, tiles
-    int ty2, parts;        // a tile in parts of ty2 rows
     double *val_grid, *val_wt_sum, *wt_sum;
     int ws_nx;
     unsigned long long *counters, *spread;
-    int *list, *list2;  // tiles that did not fit, parts of them (tile * parts + part) that did not either
-    bool all;           // all parts are taken as listed
+    int *list, *list2;  // parts of tiles that did not fit (first row, rows), rows of these that did not either;
+                        // a row is tile * ty + its place in the tile
+    bool all;           // all rows are taken as listed
 };
 
 __device__ inline void m2g_store(const M2GNodes& g, int a, int b, double wt, double vw)
@@ -269,14 +269,16 @@ __global__ __launch_bounds__(M2G_EMPTY) void m2g_count_empty(unsigned long long*
 }
 
 // A tile's markers in LDS, column of cells by column (the cells of a column are contiguous in slot
-// order): each of the M2G_COLS columns has one marker per thread, plus a spare slot per cell that ends
-// the cell's list.  28 bytes a slot, 52 KB: three workgroups per CU (256 threads and two workgroups took
-// 9.2 ms at the size below, 128 threads and four 9.5).
+// order), each column where the one before ends: its markers, at most one per thread, plus a spare slot
+// per cell that ends the cell's list.  28 bytes a slot, 40 KB: four workgroups per CU.  What bounds the
+// kernel is latency, so the workgroups in flight count (at the size below): 6.8 ms with four; 8.4 with
+// three, columns of a fixed 204 slots and 52 KB; 10.1 with five and tiles of 8 x 5 nodes.  256 threads and
+// two workgroups took 9.2, 128 threads and four, on smaller tiles, 9.5.
 #define M2G_THREADS 192
 #define M2G_COLS 9   // columns of cells, one more than of nodes
 #define M2G_ROWS 12  // most cells of a column
-#define M2G_STRIDE (M2G_THREADS + M2G_ROWS)
-#define M2G_SLOTS (M2G_COLS * M2G_STRIDE)
+#define M2G_SLOTS 1440
+#define M2G_MARGIN 1.04
 #define M2G_END 0x7fffffff
 struct M2GTile {
     double dx[M2G_SLOTS], dy[M2G_SLOTS], v[M2G_SLOTS];
@@ -284,17 +286,18 @@ struct M2GTile {
     int cell[M2G_COLS * (M2G_ROWS + 1)];  // first slot of a cell; per column one past its last cell
 };
 
-// One tile of nodes (a0..a1-1, b0..b1-1; cells a0..a1, b0..b1), by a workgroup; false if it does not fit.
+// One tile of nodes (a0..a1-1, b0..b1-1; cells a0..a1, b0..b1), by a workgroup.  0, or the rows of it that
+// should fit if it does not.
 // Each marker is read once per tile (coalesced in slot order) and its relative position computed once;
 // the per-node merges then run on LDS.  Reading 32-byte records from global memory per node instead
 // spread every load of a wave over 64 lines: 18.8 ms at 4096^2 nodes and 268 M markers, after 5.0 ms of
-// sorting the cells and 3.3 ms of writing the records, where this takes 8.3.  Of these 3.6 go to
-// the loads (2.1 GB of indices and 7.9 GB of markers with the tiles' overlap), 1.5 to the sorting and 3.3
-// to the merges (one wave of a workgroup, a chain of LDS reads).  It is bound by latency: the loads of a
-// tile are issued together, column by column without branches, and the cells are sorted by counting
-// smaller indices, all columns in step.  Merging run by run of consecutive indices (fewer choices, uneven
-// loops) took 9.8.
-__device__ inline bool m2g_tile(const M2GNodes& g, M2GTile& s, int a0, int a1, int b0, int b1)
+// sorting the cells and 3.3 ms of writing the records, where this takes 6.8.  With three workgroups per
+// CU, 3.6 of 8.4 went to the loads (2.1 GB of indices and 7.9 GB of markers with the tiles' overlap), 1.5 to
+// the sorting and 3.3 to the merges (one wave of a workgroup, a chain of LDS reads).  It is bound by
+// latency: the loads of a tile are issued together, column by column without branches, and the cells are
+// sorted by counting smaller indices, all columns in step.  Merging run by run of consecutive indices
+// (fewer choices, uneven loops) took 9.8.
+__device__ inline int m2g_tile(const M2GNodes& g, M2GTile& s, int a0, int a1, int b0, int b1)
 {
     const int t = threadIdx.x;
     const int ncx = a1 - a0 + 1, ncy = b1 - b0 + 1, nce = ncy + 1;
@@ -312,11 +315,18 @@ __device__ inline bool m2g_tile(const M2GNodes& g, M2GTile& s, int a0, int a1, i
         most = max(most, num[i]);
         total += num[i];
     }
-    if (most > M2G_THREADS) return false;  // the same for every thread
+    if (most > M2G_THREADS || total + ncx * ncy > M2G_SLOTS)  // the same for every thread
+        return max(1, min((int)(M2G_THREADS * ncy / (1.1f * most)), (int)(M2G_SLOTS * ncy / (1.1f * total + ncx * ncy))) - 1);
+    int base[M2G_COLS];  // the columns' first slots
+#pragma unroll
+    for (int i = 0; i < M2G_COLS; ++i) base[i] = i ? base[i - 1] + num[i - 1] + ncy : 0;
     if (t < ncx * nce) {
         const int i = t / nce, j = t % nce;
         const int64_t k = (int64_t)(a0 + i) * ld + b0;
-        s.cell[t] = i * M2G_STRIDE + g.off[k + j] - g.off[k] + j;
+        int first = 0;
+#pragma unroll
+        for (int u = 1; u < M2G_COLS; ++u) first = u == i ? base[u] : first;
+        s.cell[t] = first + g.off[k + j] - g.off[k] + j;
     }
     int m[M2G_COLS], place[M2G_COLS], lo[M2G_COLS], n[M2G_COLS];
     double rx[M2G_COLS], ry[M2G_COLS], rv[M2G_COLS];
@@ -334,7 +344,8 @@ __device__ inline bool m2g_tile(const M2GNodes& g, M2GTile& s, int a0, int a1, i
             rv[u] = g.val_m[m[u]];
         }
 #pragma unroll
-        for (int u = 0; u < M2G_COLS; ++u) s.idx[u * M2G_STRIDE + t] = m[u];
+        for (int u = 0; u < M2G_COLS; ++u)
+            if (t < num[u]) s.idx[base[u] + t] = m[u];
     }
     __syncthreads();
     int longest = 0;
@@ -421,7 +432,7 @@ __device__ inline bool m2g_tile(const M2GNodes& g, M2GTile& s, int a0, int a1, i
         }
         m2g_store(g, a0 + aa, b0 + bb, wt, vw);
     }
-    return true;
+    return 0;
 }
 
 __global__ __launch_bounds__(M2G_THREADS) void m2g_tiles(M2GNodes g)
@@ -429,45 +440,63 @@ __global__ __launch_bounds__(M2G_THREADS) void m2g_tiles(M2GNodes g)
     __shared__ M2GTile s;
     const int tile = xcd_band(blockIdx.x, gridDim.x);
     const int a0 = (tile / g.nty) * g.tx, b0 = (tile % g.nty) * g.ty;
-    if (!m2g_tile(g, s, a0, min(a0 + g.tx, g.gnx), b0, min(b0 + g.ty, g.gny)) && threadIdx.x == 0) {
-        if (g.parts > 1) g.list[atomicAdd(&g.counters[CNT_OVERFLOW], 1ull)] = tile;
-        else g.list2[atomicAdd(&g.spread[0], 1ull)] = tile;
+    const int a1 = min(a0 + g.tx, g.gnx), b1 = min(b0 + g.ty, g.gny);
+    const int rows = m2g_tile(g, s, a0, a1, b0, b1);
+    if (rows > 0 && threadIdx.x == 0) {
+        if (g.ty > 1) {
+            int* l = g.list + 2 * atomicAdd(&g.counters[CNT_OVERFLOW], (unsigned long long)((b1 - b0 + rows - 1) / rows));
+            for (int b = b0; b < b1; b += rows, l += 2) {
+                l[0] = tile * g.ty + b - b0;
+                l[1] = rows;
+            }
+        } else {
+            g.list2[atomicAdd(&g.spread[0], 1ull)] = tile;
+        }
     }
 }
 
-// Step 5: the tiles that did not fit, in parts.
+// Step 5: the tiles that did not fit, in parts, and these in pieces of fewer rows where they do not fit.
 __global__ __launch_bounds__(M2G_THREADS) void m2g_parts(M2GNodes g)
 {
     __shared__ M2GTile s;
-    const int n = (int)g.counters[CNT_OVERFLOW] * g.parts;
+    const int n = (int)g.counters[CNT_OVERFLOW];
     for (int w = blockIdx.x; w < n; w += gridDim.x) {
-        const int tile = g.list[w / g.parts], part = w % g.parts;
-        const int a0 = (tile / g.nty) * g.tx, b0 = (tile % g.nty) * g.ty + part * g.ty2;
-        const int b1 = min(min(b0 + g.ty2, (tile % g.nty + 1) * g.ty), g.gny);
-        if (b0 >= b1) continue;
-        if (!m2g_tile(g, s, a0, min(a0 + g.tx, g.gnx), b0, b1) && threadIdx.x == 0)
-            g.list2[atomicAdd(&g.spread[0], 1ull)] = tile * g.parts + part;
-        __syncthreads();
+        const int row = g.list[2 * w], tile = row / g.ty, row0 = (tile % g.nty) * g.ty, b0 = row0 + row % g.ty;
+        const int a0 = (tile / g.nty) * g.tx, a1 = min(a0 + g.tx, g.gnx);
+        int h = g.list[2 * w + 1];
+        const int b1 = min(min(b0 + h, row0 + g.ty), g.gny);
+        for (int b = b0; b < b1;) {
+            const int to = min(b + h, b1);
+            if (m2g_tile(g, s, a0, a1, b, to) > 0) {
+                if (h > 1) {
+                    h = (h + 1) / 2;
+                    continue;
+                }
+                if (threadIdx.x == 0) g.list2[atomicAdd(&g.spread[0], 1ull)] = tile * g.ty + b - row0;
+            }
+            b = to;
+            __syncthreads();
+        }
     }
 }
 
-// Step 5, the cells of the parts that did not fit either: each sorted in place by marker index by one workgroup, runs of
+// Step 5, the cells of the rows that did not fit: each sorted in place by marker index by one workgroup, runs of
 // M2G_RUN by counting smaller indices in LDS, longer cells by merging the runs through tmp (as long as
-// rec_idx).  A cell that several parts share is sorted by the workgroup that first takes its mark in
+// rec_idx).  A cell that several rows share is sorted by the workgroup that first takes its mark in
 // count.
 #define M2G_RUN 1024
-__device__ inline int m2g_far_parts(const M2GNodes& g)
+__device__ inline int m2g_far_rows(const M2GNodes& g)
 {
-    return g.all ? g.ntx * g.nty * g.parts : (int)g.spread[0];
+    return g.all ? g.ntx * g.nty * g.ty : (int)g.spread[0];
 }
 
-__device__ inline void m2g_far_part(const M2GNodes& g, int l, int& a0, int& a1, int& b0, int& b1)
+__device__ inline void m2g_far_row(const M2GNodes& g, int l, int& a0, int& a1, int& b0, int& b1)
 {
-    const int w = g.all ? l : g.list2[l], tile = w / g.parts;
+    const int w = g.all ? l : g.list2[l], tile = w / g.ty;
     a0 = (tile / g.nty) * g.tx;
     a1 = min(a0 + g.tx, g.gnx);
-    b0 = (tile % g.nty) * g.ty + (w % g.parts) * g.ty2;
-    b1 = min(min(b0 + g.ty2, (tile % g.nty + 1) * g.ty), g.gny);
+    b0 = (tile % g.nty) * g.ty + w % g.ty;
+    b1 = min(b0 + 1, g.gny);  // none past the grid
 }
 
 __global__ __launch_bounds__(256) void m2g_far_sort(M2GNodes g, int* count, int* tmp)
@@ -476,12 +505,12 @@ __global__ __launch_bounds__(256) void m2g_far_sort(M2GNodes g, int* count, int*
     __shared__ int s_mark;
     int* const s_idx = (int*)s_run;
     const int t = threadIdx.x;
-    const int nl = m2g_far_parts(g), most = (g.tx + 1) * (g.ty2 + 1);
+    const int nl = m2g_far_rows(g), most = (g.tx + 1) * 2;
     const int64_t ld = g.gny + 1;
     for (int64_t w = blockIdx.x; w < (int64_t)nl * most; w += gridDim.x) {
         const int c = (int)(w % most);
         int a0, a1, b0, b1;
-        m2g_far_part(g, (int)(w / most), a0, a1, b0, b1);
+        m2g_far_row(g, (int)(w / most), a0, a1, b0, b1);
         const int ncy = b1 - b0 + 1;
         if (b0 >= b1 || c >= (a1 - a0 + 1) * ncy) continue;
         const int64_t k = (int64_t)(a0 + c / ncy) * ld + b0 + c % ncy;
@@ -558,12 +587,12 @@ __global__ __launch_bounds__(256) void m2g_far_nodes(M2GNodes g)
     __shared__ int s_idx[4][4][64];
     __shared__ double s_w[4][2][256];
     const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
-    const int nl = m2g_far_parts(g), most = g.tx * g.ty2;
+    const int nl = m2g_far_rows(g), most = g.tx;
     const int64_t ld = g.gny + 1;
     for (int64_t w = (int64_t)blockIdx.x * 4 + wv; w < (int64_t)nl * most; w += (int64_t)gridDim.x * 4) {
         const int n = (int)(w % most);
         int a0, a1, b0, b1;
-        m2g_far_part(g, (int)(w / most), a0, a1, b0, b1);
+        m2g_far_row(g, (int)(w / most), a0, a1, b0, b1);
         const int na = a1 - a0;
         if (b0 >= b1 || n >= na * (b1 - b0)) continue;
         const int A = a0 + n % na + 1, B = b0 + n / na + 1;  // 1-based node
@@ -670,24 +699,33 @@ hipError_t m2g_run(M2GScratch& S, double xmin, double ymin, double* val_grid, in
     hipLaunchKernelGGL(scan_apply, dim3(nblk), dim3(SCAN_BLOCK), 0, st, S.count, ncells, S.blocksums, S.offset);
     if (nm > 0)
         hipLaunchKernelGGL(m2g_scatter, dim3(grid1d(nm, 256)), dim3(256), 0, st, S.key, S.loc, nm, S.offset, S.rec_idx);
-    M2GNodes g{S.offset, S.rec_idx, x_m, y_m, val_m, xmin, ymin, dx, dy, gnx, gny, 8, 1, 0, 0, 1, 1,
+    M2GNodes g{S.offset, S.rec_idx, x_m, y_m, val_m, xmin, ymin, dx, dy, gnx, gny, 8, 1, 0, 0,
                val_grid, val_wt_sum, wt_sum, ws_nx, S.counters, S.spread, S.loc, S.loc + nm / 2, false};
-    // Tiles of 8 columns (a row of values is half a 128-byte line), as high as fills three quarters of
-    // the slots at the mean density (markers cluster under advection), at most M2G_ROWS - 1; those that
-    // do not fit in parts of a third of their cell rows.  (A listed tile has more than M2G_THREADS markers
-    // and a marker lies in at most four tiles: both lists fit S.loc.)  Above M2G_FAR markers per cell
-    // all nodes take the kernels of step 5: 4.2 M markers in random order take 1.09 ms by tiles and
-    // 1.42 by step 5 at 72 per cell, 1.43 and 1.38 at 86 (in lattice order 0.83 and 0.73 at 76).
+    // Tiles of 8 columns (a row of values is half a 128-byte line; fewer where 9 x 2 cells do not fit), at
+    // most M2G_ROWS - 1 rows, as high as fit at the mean density: a column fills three quarters of the
+    // threads, the tile the slots with M2G_MARGIN to spare (1.15 makes tiles of 8 x 7 at 16 markers per
+    // cell: 7.5 ms at the size above against 6.8).  Advection by a continuous flow keeps lattice markers
+    // that even (512^2 to 1500^2 nodes 6 to 13% faster than with three quarters of 1836 slots); in random
+    // order about a tile in twenty goes in parts at 16 per cell (512^2: 0.61 ms, 0.60 before), and where
+    // markers cluster many do, each in as many as it needs (a normal distribution in x 0.86 ms, 0.87 before,
+    // in x and y 1.16, 1.24).  (A listed tile has more than M2G_THREADS markers and a marker lies in at most
+    // four tiles; a tile has at most M2G_ROWS - 1 parts of two words each: both lists fit S.loc.)  Above
+    // M2G_FAR markers per cell all nodes take the kernels of step 5: 4.2 M markers in random order take
+    // 0.98 ms by tiles and 1.42 by step 5 at 72 per cell, 1.43 and 1.38 at 86 (in lattice order 0.78 and 0.73 at
+    // 76).
     const double per_cell = std::max(1.0, (double)nm / ((double)gnx * gny));
     g.all = per_cell > M2G_FAR;
-    if (!g.all) g.ty = std::max(1, std::min(M2G_ROWS - 1, (int)(0.75 * M2G_THREADS / per_cell) - 1));
-    g.ty2 = std::max(1, (g.ty + 1) / 3 - 1);
-    g.parts = (g.ty + g.ty2 - 1) / g.ty2;
+    if (!g.all) {
+        const double slots = M2G_MARGIN * per_cell + 1.0;  // of a cell, the spare one included
+        const int rows = std::min(0.75 * M2G_THREADS / per_cell, M2G_SLOTS / (M2G_COLS * slots));
+        g.ty = std::max(1, std::min(M2G_ROWS - 1, rows - 1));
+        g.tx = std::min(M2G_COLS, (int)(M2G_SLOTS / ((g.ty + 1) * slots))) - 1;
+    }
     g.ntx = (gnx + g.tx - 1) / g.tx;
     g.nty = (gny + g.ty - 1) / g.ty;
     if (!g.all) {
         hipLaunchKernelGGL(m2g_tiles, dim3(g.ntx * g.nty), dim3(M2G_THREADS), 0, st, g);
-        if (g.parts > 1) hipLaunchKernelGGL(m2g_parts, dim3(768), dim3(M2G_THREADS), 0, st, g);
+        if (g.ty > 1) hipLaunchKernelGGL(m2g_parts, dim3(1024), dim3(M2G_THREADS), 0, st, g);
     }
     hipLaunchKernelGGL(m2g_far_sort, dim3(2048), dim3(256), 0, st, g, S.count, S.key);
     hipLaunchKernelGGL(m2g_far_nodes, dim3(2048), dim3(256), 0, st, g);

@@ -91,6 +91,39 @@ def test_m2g_tile_forms_bitwise_vs_oracle(gpu, nx, ny, nm, cluster):
     assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
 
 
+@pytest.mark.parametrize("nx,ny,md,dense", [
+    (65, 57, 4, 1),     # lattice markers: whole tiles with few slots left over
+    (50, 61, 5, 1),     # tiles of five rows of cells
+    (97, 90, 9, 1),     # 79 per cell: narrower tiles of one row
+    (33, 30, 7, 4),     # tiles of one row, some of which do not fit
+    (66, 43, 4, 12),    # tiles in parts, those in pieces, and rows that do not fit
+    (66, 43, 2, 45),
+    (97, 24, 1, 90),    # parts and pieces of the highest tiles
+])
+def test_m2g_packed_tiles_bitwise_vs_oracle(gpu, nx, ny, md, dense):
+    """md x md markers per cell in lattice order; `dense` times as many around one point, in random order."""
+    rng = np.random.default_rng(nx * 100 + ny)
+    dx, dy = 1.0 / (nx - 1), 0.6 / (ny - 1)
+    mx, my = md * (nx - 1), md * (ny - 1)
+    x = ((np.arange(mx)[:, None] + 0.5 + 0.5 * (rng.random((mx, my)) - 0.5)) * (dx / md)).ravel()
+    y = ((np.arange(my)[None, :] + 0.5 + 0.5 * (rng.random((mx, my)) - 0.5)) * (dy / md)).ravel()
+    if dense > 1:
+        k = int((dense - 1) * md * md * 40)
+        x = np.concatenate([x, 0.37 + 3.0 * dx * rng.standard_normal(k)])
+        y = np.concatenate([y, 0.22 + 3.0 * dy * rng.standard_normal(k)])
+        perm = rng.permutation(x.size)
+        x, y = x[perm], y[perm]
+    val = 1.0 + rng.random(x.size)
+    grid0 = np.asfortranarray(rng.random((nx, ny)))
+    vg, (vws, ws), st = m2g_gpu(0.0, 0.0, grid0, x, y, val, dx, dy, helper_shape=(nx, ny), helper_fill=3.0)
+    eg = grid0.copy(order="F")
+    evws, ews = O.zeros(nx, ny), O.zeros(nx, ny)
+    nb, ne = O.marker_to_grid(0.0, 0.0, eg, x, y, val, dx, dy, evws, ews)
+    assert np.array_equal(vg, eg)
+    assert np.array_equal(vws, evws) and np.array_equal(ws, ews)
+    assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
+
+
 def test_m2g_empty_nodes_keep_old_values(gpu):
     grid0 = np.asfortranarray(np.arange(20.0).reshape(4, 5, order="F"))
     x = np.array([0.01, 0.02])
