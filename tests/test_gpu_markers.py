@@ -124,6 +124,32 @@ def test_m2g_packed_tiles_bitwise_vs_oracle(gpu, nx, ny, md, dense):
     assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
 
 
+@pytest.mark.parametrize("extra", [0, 77, 1023])
+def test_m2g_many_markers_bitwise_vs_oracle(gpu, extra):
+    """From 2^24 markers on a thread takes four; the last workgroup has 0, 77 or 1023 of its 1024."""
+    nx, ny, nm = 901, 1000, (1 << 24) + extra
+    rng = np.random.default_rng(extra)
+    dx, dy = 1.0 / (nx - 1), 1.0 / (ny - 1)
+    # about three neighbours in a row share a cell, as in the set-up's order; some lie outside
+    x = np.repeat(rng.random(nm // 3 + 1), 3)[:nm]
+    y = np.repeat(rng.random(nm // 3 + 1), 3)[:nm]
+    x[5::1000003] = -0.5
+    y[nm - 1] = 2.0
+    val = 1.0 + rng.random(nm)
+    grid0 = np.asfortranarray(rng.random((nx, ny)))
+    vg, (vws, ws), st = m2g_gpu(0.0, 0.0, grid0, x, y, val, dx, dy, helper_shape=(nx, ny), helper_fill=3.0)
+    eg = grid0.copy(order="F")
+    evws, ews = O.zeros(nx, ny), O.zeros(nx, ny)
+    nb, ne = O.marker_to_grid(0.0, 0.0, eg, x, y, val, dx, dy, evws, ews)
+    assert np.array_equal(vg, eg)
+    assert np.array_equal(vws, evws) and np.array_equal(ws, ews)
+    assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
+    assert nb >= 17
+    keys, counts, kb = sfhip.marker_cell_keys(0.0, 0.0, nx, ny, sfhip.from_numpy(x), sfhip.from_numpy(y), dx, dy)
+    ek, ec, ekb = O.cell_keys(0.0, 0.0, nx, ny, x, y, dx, dy)
+    assert np.array_equal(keys.cpu().numpy(), ek) and np.array_equal(counts.cpu().numpy(), ec) and kb == ekb
+
+
 def test_m2g_empty_nodes_keep_old_values(gpu):
     grid0 = np.asfortranarray(np.arange(20.0).reshape(4, 5, order="F"))
     x = np.array([0.01, 0.02])
