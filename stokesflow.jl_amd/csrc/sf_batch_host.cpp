@@ -416,8 +416,6 @@ int batch_run_wide(const WideEnv& env, const sf_batch_instance* in, int n,
                 wp.n_active += 1;
             } else if (resident && !check && !last) {
                 wr.tile_start[wr.n_active] = tiles_r;
-        wp.tile_start[wp.n_active] = tiles_p;
-        if (wp.n_active) HIPCHK(launch_wide_pipe(wp, s));
                 wr.slot_inst[wr.n_active] = r.id;
                 wr.slot_pf[wr.n_active] = par | (r.k << 1);
                 tiles_r += wide_resident_tiles(plan, a.nx, a.ny, r.k);

@@ -289,3 +289,33 @@ def test_wide_default_passes(gpu, sizes, cap):
         assert o["err"] == pytest.approx(st["err"], rel=1e-12, abs=0.0)
         for k in OUT:
             assert np.array_equal(sfhip.to_numpy(G[k]), exp[k]), (nx, ny, k)
+
+
+def kernel_launches(fn, name):
+    """Launches of kernels whose name holds ``name`` while ``fn`` runs."""
+    from torch.profiler import ProfilerActivity, profile
+
+    with profile(activities=[ProfilerActivity.CUDA, ProfilerActivity.CPU]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    kernels = [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    assert any("sf::" in k for k in kernels), sorted(set(kernels))  # the library's launches are recorded
+    return sum(name in k for k in kernels)
+
+
+def test_wide_pipelined_pass_once_per_step(gpu):
+    """Every instance runs passes of seven iterations to its cap (71: ten passes and the last iteration);
+    those with caps 24, 33 and 47 meet it with shorter passes beside the others' pipelined ones, which
+    then still run once in that step."""
+    caps = [(256, 257, 71)] * 15 + [(131, 250, c) for c in (24, 33, 47)]
+    insts = [(nx, ny, cap, cases.smooth_state(nx, ny, seed=80 + k)) for k, (nx, ny, cap) in enumerate(caps)]
+    probs = [problem(S, nx, ny, 1.0 / (nx - 1), 1.0 / (ny - 1), iterMax=cap) for nx, ny, cap, S in insts]
+    outs = []
+    n = kernel_launches(lambda: outs.extend(sfhip.solveStokes_batched([p for p, _ in probs], mode="wide")),
+                        "wide_ptp_kernel")
+    assert n == 10, n
+    for (nx, ny, cap, S), (_, G), o in list(zip(insts, probs, outs))[-4:]:
+        st, exp = single(S, nx, ny, 1.0 / (nx - 1), 1.0 / (ny - 1), iterMax=cap)
+        assert o["niter"] == st["niter"] == cap
+        for k in OUT:
+            assert np.array_equal(sfhip.to_numpy(G[k]), exp[k]), (nx, ny, k)
