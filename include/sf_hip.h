@@ -236,6 +236,10 @@ int sf_solve_stokes_refined(sf_ctx *ctx, double *P, double *Vx_pad, double *Vy_p
  * separated by a grid barrier; no host synchronisation, so it can be captured
  * (sf_graph_*).  A barrier wait longer than the limit (5 s unless sf_set_grid_wait_limit sets
  * another; workgroups not all resident) ends the launch and the call returns SF_ERR_HIP.
+ * Grid solves and sf_graph_step / grid-form sf_ensemble_step calls of several threads on one GPU
+ * take turns where their workgroups together number more than its CUs (two of more than about 100^2
+ * nodes each), so they never hold each other up to that limit; processes that share a GPU know
+ * nothing of each other and must not run them at the same time.
  * With precision 1 (WIDE only) every instance is solved as sf_solve_stokes_refined solves it,
  * with one launch per FP32 sweep of all active instances.
  * In FP64 every PT iteration is bit-identical to sf_solve_stokes.  outs[i] gets instance i's dt_new,

@@ -217,6 +217,30 @@ GridShape grid_launch_shape(const BatchInstance& d, int k)
     return GridShape{nwg, waves, k, 0};
 }
 
+void GridHold::enter(int nwg, hipStream_t s)
+{
+    static GridGate gates[16];
+    int dev = 0, cus = 0;
+    if (hipStreamGetDevice(s, &dev) != hipSuccess || dev < 0) dev = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    gate = &gates[dev % 16];
+    n = nwg;
+    stream = s;
+    gate->enter(n, cus);
+}
+
+void GridHold::leave()
+{
+    if (gate) gate->leave(n);
+    gate = nullptr;
+}
+
+GridHold::~GridHold()
+{
+    if (gate) (void)hipStreamSynchronize(stream);
+    leave();
+}
+
 }  // namespace sf
 
 extern "C" int sf_set_grid_wait_limit(double seconds)
@@ -1060,8 +1084,10 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         const int k = (prm && prm->depth >= 1 && prm->depth <= 3) ? prm->depth : 0;
         std::vector<GridShape> shape((size_t)n);
         size_t exch = 0;
+        int nwg = 0;
         for (int i = 0; i < n; ++i) {
             shape[(size_t)i] = grid_launch_shape(host[(size_t)i], k);
+            nwg = std::max(nwg, shape[(size_t)i].nwg);
             if (shape[(size_t)i].r) exch = std::max(exch, grid_exchange_doubles(in[i].nx, in[i].ny));
         }
         rc = grid_reserve(c, n, exch);
@@ -1069,6 +1095,8 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         HIPCHK(hipMemsetAsync(c->g_sync, 0, sizeof(unsigned long long) * GRID_SYNC_WORDS * (size_t)n, s));
         const double wait_s = grid_wait_seconds();
         const uint64_t wait_ticks = grid_wait_limit();
+        GridHold hold;
+        hold.enter(nwg, s);
         for (int qi = 0; qi < n; ++qi) {
             const int i = order[(size_t)qi];
             const GridShape& gs = shape[(size_t)i];
@@ -1081,6 +1109,7 @@ extern "C" int sf_solve_stokes_batched(sf_ctx* c, const sf_batch_instance* in, i
         HIPCHK(hipMemcpyAsync(sync.data(), c->g_sync, sizeof(unsigned long long) * GRID_SYNC_WORDS * (size_t)n,
                               hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
+        hold.leave();
         for (int i = 0; i < n; ++i)
             if (sync[(size_t)GRID_SYNC_WORDS * i + GRID_SYNC_STICKY])
                 return set_err(SF_ERR_HIP, "%s: instance %d: a grid barrier wait exceeded %g s (workgroups not all resident?)",

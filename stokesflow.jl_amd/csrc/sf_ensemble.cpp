@@ -337,6 +337,12 @@ extern "C" int sf_ensemble_step(sf_ensemble* e, int n_steps, sf_solve_out* outs,
     HIPCHK(hipEventRecord(e->ev, e->c->stream));
     HIPCHK(hipStreamWaitEvent(e->stream, e->ev, 0));
     std::vector<BatchResult> res;
+    GridHold hold;
+    if (e->grid && n_steps > 0) {
+        int nwg = 0;
+        for (const GridShape& gs : e->gshape) nwg = std::max(nwg, gs.nwg);
+        hold.enter(nwg, e->stream);
+    }
     for (int k = 0; k < n_steps; ++k) {
         if (!e->wide) {
             if (e->use_graph)
@@ -373,6 +379,7 @@ extern "C" int sf_ensemble_step(sf_ensemble* e, int n_steps, sf_solve_out* outs,
     HIPCHK(hipMemcpyAsync(e->hcnt, e->cnt, sizeof(unsigned long long) * ENS_CNT * (size_t)e->n, hipMemcpyDeviceToHost,
                           e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
+    hold.leave();
     const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
     if (n_steps > 0 && e->grid)
         for (int i = 0; i < e->n; ++i)

@@ -14,6 +14,7 @@
 #include <utility>
 #include <vector>
 
+#include "sf_grid_gate.h"
 #include "sf_internal.h"
 
 namespace sf {
@@ -90,6 +91,23 @@ struct GridShape {
     int k, r;        // GridArgs
 };
 GridShape grid_launch_shape(const BatchInstance& d, int k);
+// A call's place at the device's GridGate: from enter(), before its first grid-mode launch on s, of at most
+// nwg workgroups at a time, until leave(), after s has been waited for.  A call that ends without leave()
+// waits for s first.
+class GridHold {
+public:
+    GridHold() = default;
+    GridHold(const GridHold&) = delete;
+    GridHold& operator=(const GridHold&) = delete;
+    ~GridHold();
+    void enter(int nwg, hipStream_t s);
+    void leave();
+
+private:
+    GridGate* gate = nullptr;
+    int n = 0;
+    hipStream_t stream = nullptr;
+};
 BatchInstance batch_descriptor(const sf_batch_instance& a, int rows, double* q, const double* dt_dev,
                                const BatchShape& sh = BatchShape());
 std::vector<int> batch_order(const std::vector<std::pair<int, int>>& dims);

@@ -176,3 +176,36 @@ def test_grid_wait_limit_error_path(gpu):
     outs = sfhip.solveStokes_batched([pb], mode="grid")
     torch.cuda.synchronize()
     check_against_single([(nx, ny, S, dx, dy)], outs, [G], iterMax=10)
+
+
+def test_step_graphs_of_two_threads(gpu):
+    """Captured steps of 200 and 231 workgroups replayed from two threads at once: either fits the chip, both
+    together do not, so they take turns; the results are those of replays one after the other."""
+    import threading
+
+    sizes = [(200, 200), (301, 257)]
+    ms = [[member(nx, ny, 800 + k) for _ in range(2)] for k, (nx, ny) in enumerate(sizes)]
+    graphs = [[sfhip.StepGraph(m["state"], m["x_m"], m["y_m"], m["rho_m"], m["mu_m"], m["dx"], m["dy"], 0.0, g_y=1.0,
+                               eps=1e-5) for m in pair] for pair in ms]
+    torch.cuda.synchronize()
+    got, start = [[], []], threading.Barrier(2)
+
+    def replay(k):
+        start.wait(30)
+        try:
+            for _ in range(4):
+                got[k].append(graphs[k][0].step(2)[0])
+        except Exception as e:  # shown by the comparison below
+            got[k].append(repr(e))
+
+    ts = [threading.Thread(target=replay, args=(k,)) for k in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(100)
+    for k in range(2):
+        assert got[k] == [graphs[k][1].step(2)[0] for _ in range(4)]
+        torch.cuda.synchronize()
+        same(*ms[k])
+        for g in graphs[k]:
+            g.close()
