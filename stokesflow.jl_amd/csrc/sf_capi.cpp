@@ -819,7 +819,9 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
         const int explicit_fuse = c->fuse, explicit_rows = c->pair_rows;
         c->fuse64 = c->rows64 = c->fuse = c->pair_rows = 0;
         const int n_plan = std::max(28, (iters + 27) / 28 * 28);
-        const int r = time_shape(PT_PLAN_MAX_K, n_plan, &plan_us);
+        // (14 iterations first: a shorter run of a pipelined plan takes the one-wave passes, run_fixed, and
+        // the plan's first launch, which loads its code, 0.4 ms, would be timed)
+        const int r = time_shape(2 * PT_PLAN_MAX_K, n_plan, &plan_us);
         c->fuse = explicit_fuse;
         c->pair_rows = explicit_rows;
         return r;

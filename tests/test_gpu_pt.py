@@ -454,3 +454,19 @@ def test_refined_default_passes_bitwise(gpu, nx, ny, cap, rebase):
     assert s1["n_fp32_iter"] == s2["n_fp32_iter"]
     for k in a1:
         assert np.array_equal(a1[k], a2[k], equal_nan=True), k
+
+
+def test_autotune_warms_the_size_default(gpu):
+    """The autotuner times 56 iterations of the size default's pass (pipelined at 1024^2) after two
+    untimed passes of it, so that the first launch of the kernel is not timed."""
+    n = 1024
+    sfhip.set_pt_fusion(n, n, 0, 0)
+    sfhip.time_passes(n, n, True)
+    try:
+        sfhip.autotune_pt(n, n, iters=30)
+        sevens = [t["launches"] for t in sfhip.pass_times(n, n) if t["iters_per_launch"] == 7]
+    finally:
+        sfhip.time_passes(n, n, False)
+        sfhip.set_pt_tuning(n, n, 0, 0, -1)
+        sfhip.set_pt_fusion(n, n, 0, 0)
+    assert sevens == [2 + 8], sevens
