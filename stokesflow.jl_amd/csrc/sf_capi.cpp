@@ -777,7 +777,6 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
     };
     sf_pt_tuning bestv{}, best_all{};
     bestv.us_per_iter = 1e300;
-    double plan_us = 1e300;
     // first the shapes of the one-iteration kernel; every loop ends at the first error
     const int rc = [&]() -> int {
         c->fuse64 = 1;
@@ -821,10 +820,14 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
         const int n_plan = std::max(28, (iters + 27) / 28 * 28);
         // (14 iterations first: a shorter run of a pipelined plan takes the one-wave passes, run_fixed, and
         // the plan's first launch, which loads its code, 0.4 ms, would be timed)
-        const int r = time_shape(2 * PT_PLAN_MAX_K, n_plan, &plan_us);
+        sf_pt_tuning t{0, 1, -1, 0, 0.0};
+        const int r = time_shape(2 * PT_PLAN_MAX_K, n_plan, &t.us_per_iter);
         c->fuse = explicit_fuse;
         c->pair_rows = explicit_rows;
-        return r;
+        if (r) return r;
+        record(t);
+        if (t.us_per_iter < best_all.us_per_iter) best_all = t;
+        return SF_OK;
     }();
     (void)hipStreamSynchronize(s);
     release();
@@ -842,7 +845,6 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
     // the FP64 passes only: the FP32 sweeps of the refined solver keep their own defaults
     c->fuse64 = best_all.iters_per_launch;
     c->rows64 = best_all.iters_per_launch > 1 ? best_all.rows : 0;
-    if (plan_us < best_all.us_per_iter) c->fuse64 = c->rows64 = 0;
     if (best) *best = best_all;
     if (n_table) *n_table = nt;
     return SF_OK;

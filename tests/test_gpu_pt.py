@@ -470,3 +470,28 @@ def test_autotune_warms_the_size_default(gpu):
         sfhip.set_pt_tuning(n, n, 0, 0, -1)
         sfhip.set_pt_fusion(n, n, 0, 0)
     assert sevens == [2 + 8], sevens
+
+
+def launches_after_tuning(nx, ny):
+    """(best, table) of the autotuner, and the passes that 28 iterations then take."""
+    best, table = sfhip.autotune_pt(nx, ny, iters=30)
+    S = cases.smooth_state(nx, ny, seed=6)
+    sfhip.time_passes(nx, ny, True)
+    run_gpu_iterations(S, nx, ny, 28, 1.0, 1.0 / (nx - 1), 1.0 / (ny - 1), 0.01)
+    return best, table, [(t["iters_per_launch"], t["launches"]) for t in sfhip.pass_times(nx, ny)]
+
+
+@pytest.mark.parametrize("nx,ny", [(63, 47), (900, 801)])
+def test_autotune_best_is_what_is_set(gpu, nx, ny):
+    """The size default is in the table (iters_per_launch 0) and `best` names what later iterations take."""
+    try:
+        best, table, launches = launches_after_tuning(nx, ny)
+    finally:
+        sfhip.time_passes(nx, ny, False)
+        sfhip.set_pt_tuning(nx, ny, 0, 0, -1)
+        sfhip.set_pt_fusion(nx, ny, 0, 0)
+    assert [t["rows"] for t in table if t["iters_per_launch"] == 0] == [0]
+    assert best["us_per_iter"] == min(t["us_per_iter"] for t in table)
+    k = best["iters_per_launch"] or 7  # the default's passes of seven at both sizes
+    exp = {j: n for j, n in ((k, 28 // k), (28 % k, 1)) if j > 1}  # single iterations are not timed
+    assert dict(launches) == exp, (best, launches)
