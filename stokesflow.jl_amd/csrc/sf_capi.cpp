@@ -244,8 +244,8 @@ static int ctx_pt_buffers(sf_ctx* c, bool pairs, PTBuffers* b)
 // size default.
 static int ctx_pt_loop(sf_ctx* c, PTLoop* L, double* Vx_s, double* Vy_s, double* P, double* dVx, double* dVy)
 {
-    const int fuse = c->fuse64 > 0 ? c->fuse64 : c->fuse;
-    const int rows = c->fuse64 > 0 ? c->rows64 : c->pair_rows;
+    const int fuse = c->fuse64 == 0 ? c->fuse : std::max(c->fuse64, 0);
+    const int rows = c->fuse64 == 0 ? c->pair_rows : c->rows64;
     PTBuffers b{};
     const int rc = ctx_pt_buffers(c, fuse != 1, &b);
     if (rc) return rc;
@@ -636,8 +636,8 @@ extern "C" int sf_solve_stokes(sf_ctx* c, double* P, double* Vx_pad, double* Vy_
     int rc = check_ctx(c, nx, ny, "sf_solve_stokes");
     if (rc) return rc;
     // the autotuner's FP64 choice, else the explicit setting, else the size default
-    const int fuse = c->fuse64 > 0 ? c->fuse64 : c->fuse;
-    const int rows = c->fuse64 > 0 ? c->rows64 : c->pair_rows;
+    const int fuse = c->fuse64 == 0 ? c->fuse : std::max(c->fuse64, 0);
+    const int rows = c->fuse64 == 0 ? c->pair_rows : c->rows64;
     PTBuffers b{};
     rc = ctx_pt_buffers(c, fuse != 1, &b);
     if (rc) return rc;
@@ -815,15 +815,13 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
             }
         }
         // last the size default's pass, which is kept where none of the table is faster
-        const int explicit_fuse = c->fuse, explicit_rows = c->pair_rows;
-        c->fuse64 = c->rows64 = c->fuse = c->pair_rows = 0;
+        c->fuse64 = -1;
+        c->rows64 = 0;
         const int n_plan = std::max(28, (iters + 27) / 28 * 28);
         // (14 iterations first: a shorter run of a pipelined plan takes the one-wave passes, run_fixed, and
         // the plan's first launch, which loads its code, 0.4 ms, would be timed)
         sf_pt_tuning t{0, 1, -1, 0, 0.0};
         const int r = time_shape(2 * PT_PLAN_MAX_K, n_plan, &t.us_per_iter);
-        c->fuse = explicit_fuse;
-        c->pair_rows = explicit_rows;
         if (r) return r;
         record(t);
         if (t.us_per_iter < best_all.us_per_iter) best_all = t;
@@ -843,7 +841,7 @@ extern "C" int sf_ctx_autotune_pt(sf_ctx* c, int iters, const double* P_in, cons
     c->depth = bestv.depth;
     c->max_waves = bestv.max_waves;
     // the FP64 passes only: the FP32 sweeps of the refined solver keep their own defaults
-    c->fuse64 = best_all.iters_per_launch;
+    c->fuse64 = best_all.iters_per_launch ? best_all.iters_per_launch : -1;
     c->rows64 = best_all.iters_per_launch > 1 ? best_all.rows : 0;
     if (best) *best = best_all;
     if (n_table) *n_table = nt;

@@ -284,7 +284,7 @@ struct sf_ctx {
     int max_waves = -1; // 0 persistent (resident slots), > 0 cap, < 0 one wave per tile
     int fuse = 0;       // sf_ctx_set_pt_fusion: iterations / FP32 sweeps per pass (0 size default, 1..5)
     int pair_rows = 0;  // rows per tile of the multi-iteration passes; 0 = size default
-    int fuse64 = 0;     // autotuner's choice for the FP64 passes only (0: none; then fuse / pair_rows apply)
+    int fuse64 = 0;     // autotuner's choice for the FP64 passes only (0: none, then fuse / pair_rows apply; -1: the size default)
     int rows64 = 0;
     double *dvx_b = nullptr, *dvy_b = nullptr;  // second dVx/dVy (two-iteration pass)
     sf::PassTimer timer;  // sf_ctx_time_passes

@@ -495,3 +495,23 @@ def test_autotune_best_is_what_is_set(gpu, nx, ny):
     k = best["iters_per_launch"] or 7  # the default's passes of seven at both sizes
     exp = {j: n for j, n in ((k, 28 // k), (28 % k, 1)) if j > 1}  # single iterations are not timed
     assert dict(launches) == exp, (best, launches)
+
+
+def test_autotune_replaces_explicit_passes(gpu):
+    """The tuner's choice replaces an explicit number of iterations per launch also where it is the size
+    default; an explicit setting afterwards replaces the tuner's choice."""
+    nx, ny = 900, 801
+    try:
+        sfhip.set_pt_fusion(nx, ny, 2, 0)
+        best, _, launches = launches_after_tuning(nx, ny)
+        k = best["iters_per_launch"] or 7
+        assert dict(launches) == {j: n for j, n in ((k, 28 // k), (28 % k, 1)) if j > 1}, (best, launches)
+        sfhip.set_pt_fusion(nx, ny, 2, 0)
+        S = cases.smooth_state(nx, ny, seed=6)
+        sfhip.time_passes(nx, ny, True)
+        run_gpu_iterations(S, nx, ny, 28, 1.0, 1.0 / (nx - 1), 1.0 / (ny - 1), 0.01)
+        assert [(t["iters_per_launch"], t["launches"]) for t in sfhip.pass_times(nx, ny)] == [(2, 14)]
+    finally:
+        sfhip.time_passes(nx, ny, False)
+        sfhip.set_pt_tuning(nx, ny, 0, 0, -1)
+        sfhip.set_pt_fusion(nx, ny, 0, 0)
