@@ -319,3 +319,18 @@ def test_wide_pipelined_pass_once_per_step(gpu):
         assert o["niter"] == st["niter"] == cap
         for k in OUT:
             assert np.array_equal(sfhip.to_numpy(G[k]), exp[k]), (nx, ny, k)
+
+
+def test_batch_autotune_warms_the_size_defaults(gpu):
+    """The tuner runs the size defaults on the whole batch once untimed and once timed before it
+    compares a choice with them: twice the launches of one such run (240 iterations)."""
+    insts = [cases.smooth_state(64, 64, seed=120 + k) for k in range(4)]
+    problems = [problem(S, 64, 64, 1.0 / 63, 1.0 / 63, iterMax=240)[0] for S in insts]
+    sfhip.clear_batched_tuning()
+    one = kernel_launches(lambda: sfhip.solveStokes_batched(problems, mode="wide"), "wide_ptr_kernel")
+    assert one > 0
+    try:
+        n = kernel_launches(lambda: sfhip.autotune_batched(problems, iters=12), "wide_ptr_kernel")
+    finally:
+        sfhip.clear_batched_tuning()
+    assert n == 2 * one, (n, one)
