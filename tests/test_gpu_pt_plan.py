@@ -46,3 +46,16 @@ def test_size_default_passes_extreme_viscosity(gpu, nx, ny, log2_mu):
     for k in STATE:
         S[k][:] = 0.0
     _compare(S, nx, ny, 15)
+
+
+def test_pipelined_pass_4096_bitwise(gpu):
+    """The kernel of 4096^2 solves at that size: two pipelined passes of seven iterations and one of four
+    (a run of less than two whole passes keeps the one-wave ones)."""
+    n = 4096
+    sfhip.time_passes(n, n, True)
+    try:
+        _compare(cases.random_state(n, n, seed=4097, scale=1e-3, contrast=4.0), n, n, 18)
+        launches = sfhip.pass_times(n, n)
+    finally:
+        sfhip.time_passes(n, n, False)
+    assert sorted((t["precision"], t["iters_per_launch"], t["launches"]) for t in launches) == [(0, 4, 1), (0, 7, 2)]
