@@ -247,7 +247,8 @@ extern "C" int sf_ensemble_create(sf_ctx* c, const sf_step_args* members, int n,
     e->dt.resize((size_t)n);
     std::vector<std::pair<int, int>> dims((size_t)n);
     for (int i = 0; i < n; ++i) {
-        const BatchShape sh = e->grid ? BatchShape() : batch_shape(c, members[i].nx, members[i].ny);
+        BatchShape sh = e->grid ? BatchShape() : batch_shape(c, members[i].nx, members[i].ny);
+        if (!e->wide && !e->grid && sh.rows3 <= 0) sh.rows3 = persistent_rows(members[i].nx, members[i].ny, n);
         e->desc[(size_t)i] = batch_descriptor(bi[(size_t)i], rows, e->pool + off[(size_t)i], e->wide ? nullptr : &e->res[i].dt_new,
                                               sh);
         dims[(size_t)i] = {members[i].nx, members[i].ny};

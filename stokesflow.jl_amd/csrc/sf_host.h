@@ -86,6 +86,7 @@ struct BatchTune {
     BatchShape sh;
 };
 BatchShape batch_shape(const sf_ctx* c, int nx, int ny);
+int persistent_rows(int nx, int ny, int n);
 struct GridShape {
     int nwg, waves;  // workgroups, waves per workgroup
     int k, r;        // GridArgs

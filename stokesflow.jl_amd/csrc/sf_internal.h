@@ -77,7 +77,7 @@ int pt2_default_rows(int nx, int ny);
 // p.seg <= 0: ptk_default_rows).
 hipError_t launch_pt_multi(const PTParams& p, int k, hipStream_t s);
 // tile height of a k-iteration pass (k >= 3) when `copies` grids of this size share the launch
-int ptk_default_rows(int k, int nx, int ny);
+int ptk_default_rows(int k, int nx, int ny, int copies = 1);
 // k = 5, 6 or 7 PT iterations per pass, pipelined over the waves of a workgroup (sf_ptp_tile.h), in
 // tiles of `rows` rows.
 hipError_t launch_pt_pipe(const PTParams& p, int k, int rows, hipStream_t s);
