@@ -209,3 +209,24 @@ def test_step_graphs_of_two_threads(gpu):
         same(*ms[k])
         for g in graphs[k]:
             g.close()
+
+
+def test_grid_checks_of_narrow_grids(gpu):
+    """A 3 x 1000 grid checks every 15 iterations: the default's checks, with up to 16 waves per workgroup,
+    cost no more than those of the one-wave passes (it takes 0.8 of their time; 1.5 where every
+    wave read every other's partials)."""
+    import time
+
+    nx, ny = 3, 1000
+    S = cases.smooth_state(nx, ny, seed=640)
+    best = {}
+    for depth in (0, 3):
+        pb, G = problem(S, nx, ny, 1.0 / (nx - 1), 1.0 / (ny - 1), iterMax=600, eps=1e-300)
+        times = []
+        for _ in range(6):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            sfhip.solveStokes_batched([pb], mode="grid", depth=depth)
+            times.append(time.perf_counter() - t0)
+        best[depth] = min(times[1:])
+    assert best[0] < 1.2 * best[3], best
