@@ -211,8 +211,13 @@ GridShape grid_launch_shape(const BatchInstance& d, int k)
         if (plan.kind == PT_PLAN_RESIDENT && (int64_t)d.nx * d.ny <= GRID_RESIDENT_NODES) {
             const int out = 64 - 2 * plan.k, seg = plan.waves * plan.r - 2 * plan.k;
             const int64_t t = (int64_t)((d.nx - 1 + out - 1) / out) * ((d.ny + seg - 1) / seg);
-            const int nwg = (int)std::min<int64_t>(t, grid_capacity(plan.k, plan.r, plan.waves));
-            if (nwg > 0) return GridShape{nwg, plan.waves, plan.k, plan.r};
+            const int cap = grid_capacity(plan.k, plan.r, plan.waves);
+            // Flat grids whose tiles are not all resident: a one-wave tile marches over the whole height, a
+            // resident one is mostly halo rows (us per iteration, one-wave passes and resident: 50000x4 7.0,
+            // 13.5; 100000x8 10.4, 15.9; 20000x11 6.5, 7.0, but 20000x16 7.8, 6.6; with more than three tiles per
+            // CU 50000x16 10.4, 11.3).
+            const bool flat = t > cap && d.ny < (t > 3 * cap ? 24 : 12);
+            if (cap > 0 && !flat) return GridShape{(int)std::min<int64_t>(t, cap), plan.waves, plan.k, plan.r};
         }
         k = 3;
     }

@@ -13,7 +13,7 @@ import sfhip
 from oracle import sf_oracle as O
 
 import cases
-from test_gpu_batch import OUT, plume_instance, problem, single
+from test_gpu_batch import OUT, kernel_launches, plume_instance, problem, single
 from test_gpu_ensemble import member, same
 
 pytestmark = pytest.mark.gpu
@@ -230,3 +230,16 @@ def test_grid_checks_of_narrow_grids(gpu):
             times.append(time.perf_counter() - t0)
         best[depth] = min(times[1:])
     assert best[0] < 1.2 * best[3], best
+
+
+@pytest.mark.parametrize("nx,ny,resident", [(50000, 4, False), (20000, 11, False), (20000, 16, True), (50000, 16, False),
+                                            (900, 11, True), (4, 20000, True)])
+def test_grid_mode_flat_grids(gpu, nx, ny, resident):
+    """Flat grids with more tiles than CUs take the one-wave passes."""
+    S = cases.smooth_state(nx, ny, seed=650)
+    dx, dy = 1.0 / (nx - 1), 1.0 / (ny - 1)
+    pb, G = problem(S, nx, ny, dx, dy, iterMax=47)
+    outs = []
+    n = kernel_launches(lambda: outs.extend(sfhip.solveStokes_batched([pb], mode="grid")), "grid_solve_kernel<3, 0>")
+    assert n == (0 if resident else 1)
+    check_against_single([(nx, ny, S, dx, dy)], outs, [G], iterMax=47)
