@@ -200,7 +200,7 @@ struct PTLoop {
         plan = PTPlan{};
         if (fuse == 0 && pass_rows == 0) {
             plan = pt_plan(nx, ny);
-            kmax = plan.k;
+            if (plan.kind != PT_PLAN_NONE) kmax = plan.k;
         }
     }
     // One iteration (flags: check-iteration outputs); dV in place.

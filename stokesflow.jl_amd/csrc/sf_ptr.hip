@@ -46,6 +46,8 @@ static const Shape shapes[] = {{8, 1, 0.6, 0.54},  {12, 1, 1.1, 0.61}, {16, 1, 1
 
 static const double pipe_step[3] = {0.55, 0.72, 0.94};  // us per row step, workgroups per CU
 
+#define WIDE_PIPE_MARGIN 1.15  // see wide_plan
+
 static int wide_pipe_rows(int ny, int h)
 {
     const int nseg = (ny + h - 1) / h;
@@ -111,6 +113,14 @@ PTPlan pt_plan(int nx, int ny)
             best = PTPlan{PT_PLAN_PIPE, k, rows, 0, 0};
         }
     }
+    // Flat grids: a wave of the one-wave passes of four iterations marches over the whole height.  Its row
+    // step takes 2.2 us with two waves per SIMD and 1.6 with one (ptk_default_rows); the pipelined
+    // model is 15% short there (WIDE_PIPE_MARGIN).  us per iteration, one-wave and the plan: 100000x4
+    // 6.9, 9.2; 100000x8 8.9, 9.9; 250000x6 16.5, 20.1; 50000x4 5.2, 5.8; but 50000x11 7.7, 6.7.
+    const int ow_rows = ptk_default_rows(4, nx, ny);
+    const double waves = (double)((nx - 1 + 55) / 56) * ((ny + ow_rows - 1) / ow_rows);
+    const double ow_us = (2.5 + (ow_rows + 7) * (waves <= 4 * cus ? 1.6 : 2.2 * std::max(1.0, waves / (8 * cus)))) / 4;
+    if (ow_us < best_us * (best.kind == PT_PLAN_PIPE ? WIDE_PIPE_MARGIN : 1.0)) best = PTPlan{};
     return best;
 }
 
@@ -125,7 +135,6 @@ PTPlan pt_plan(int nx, int ny)
 // before): one 64^2 1.9, 3.1, 3.1; 64 x 64^2 7.2, 8.1, 9.9; 4 x 100x90 2.1, 3.2, 3.4; 16 x 256^2 11.2, 8.5, 11.2;
 // 64 x 256^2 48, 32, 43; 8 x 512^2 17.6, 12.9, 18.0; one 2048^2 34, 24, 32.  The pipelined model gains
 // WIDE_PIPE_MARGIN too much on sets near the line (it has the row steps but not the pipeline's start).
-#define WIDE_PIPE_MARGIN 1.15
 WidePlan wide_plan(const int* nx, const int* ny, int n, int* k, int* rows)
 {
     const int cus = 256;

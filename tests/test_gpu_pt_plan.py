@@ -59,3 +59,15 @@ def test_pipelined_pass_4096_bitwise(gpu):
     finally:
         sfhip.time_passes(n, n, False)
     assert sorted((t["precision"], t["iters_per_launch"], t["launches"]) for t in launches) == [(0, 4, 1), (0, 7, 2)]
+
+
+def test_flat_grid_bitwise(gpu):
+    """A flat grid of 1,786 strips keeps the one-wave passes of four iterations."""
+    nx, ny = 100000, 5
+    sfhip.time_passes(nx, ny, True)
+    try:
+        _compare(cases.random_state(nx, ny, seed=11), nx, ny, 19)
+        launches = sfhip.pass_times(nx, ny)
+    finally:
+        sfhip.time_passes(nx, ny, False)
+    assert sorted((t["iters_per_launch"], t["launches"]) for t in launches) == [(3, 1), (4, 4)]

@@ -20,6 +20,7 @@ int main(int argc, char** argv)
     int a, b, c;
     while (std::scanf("%31s %d %d %d", what, &a, &b, &c) == 4) {
         if (!std::strcmp(what, "persistent")) std::printf("%d\n", persistent_rows(a, b, c));
+        if (!std::strcmp(what, "plan")) std::printf("%d\n", pt_plan(a, b).kind);
     }
     return 0;
 }
@@ -60,3 +61,13 @@ def test_persistent_rows(shapes):
     few = [(64, 3, 2), (20, 3000, 8), (256, 256, 4), (256, 256, 63), (64, 64, 1), (455, 400, 24)]
     got = shapes([f"persistent {nx} {ny} {n}" for nx, ny, n in [*many, *few]])
     assert [r[0] for r in got] == [*many.values(), *(wave_rounds_rows(3, *c) for c in few)]
+
+
+def test_flat_grids_keep_one_wave_passes(shapes):
+    """pt_plan's kinds (0 one-wave, 1 resident, 2 pipelined): one-wave only on flat grids of many strips."""
+    one_wave = [(50000, 4), (100000, 3), (100000, 8), (250000, 6)]
+    others = [(64, 64), (700, 700), (1024, 1024), (4096, 4096), (20000, 3), (20000, 8), (50000, 11), (8, 100000), (250000, 24),
+              (16384, 16384)]
+    kinds = [r[0] for r in shapes([f"plan {nx} {ny} 0" for nx, ny in one_wave + others])]
+    assert kinds[:len(one_wave)] == [0] * len(one_wave)
+    assert 0 not in kinds[len(one_wave):]
