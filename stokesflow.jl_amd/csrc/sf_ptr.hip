@@ -113,14 +113,15 @@ PTPlan pt_plan(int nx, int ny)
             best = PTPlan{PT_PLAN_PIPE, k, rows, 0, 0};
         }
     }
-    // Flat grids: a wave of the one-wave passes of four iterations marches over the whole height.  Its row
-    // step takes 2.2 us with two waves per SIMD and 1.6 with one (ptk_default_rows); the pipelined
+    // Flat grids: a wave of the one-wave passes of four iterations marches over the whole height (from 16
+    // rows on the two are equal within 5%).  Its row step takes 2.2 us with two waves per SIMD and 1.6 with one (ptk_default_rows); the pipelined
     // model is 15% short there (WIDE_PIPE_MARGIN).  us per iteration, one-wave and the plan: 100000x4
     // 6.9, 9.2; 100000x8 8.9, 9.9; 250000x6 16.5, 20.1; 50000x4 5.2, 5.8; but 50000x11 7.7, 6.7.
-    const int ow_rows = ptk_default_rows(4, nx, ny);
-    const double waves = (double)((nx - 1 + 55) / 56) * ((ny + ow_rows - 1) / ow_rows);
-    const double ow_us = (2.5 + (ow_rows + 7) * (waves <= 4 * cus ? 1.6 : 2.2 * std::max(1.0, waves / (8 * cus)))) / 4;
-    if (ow_us < best_us * (best.kind == PT_PLAN_PIPE ? WIDE_PIPE_MARGIN : 1.0)) best = PTPlan{};
+    if (ny < 16) {
+        const double waves = (nx - 1 + 55) / 56;
+        const double ow_us = (2.5 + (ny + 7) * (waves <= 4 * cus ? 1.6 : 2.2 * std::max(1.0, waves / (8 * cus)))) / 4;
+        if (ow_us < best_us * (best.kind == PT_PLAN_PIPE ? WIDE_PIPE_MARGIN : 1.0)) best = PTPlan{};
+    }
     return best;
 }
 

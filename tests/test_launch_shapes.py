@@ -67,7 +67,7 @@ def test_flat_grids_keep_one_wave_passes(shapes):
     """pt_plan's kinds (0 one-wave, 1 resident, 2 pipelined): one-wave only on flat grids of many strips."""
     one_wave = [(50000, 4), (100000, 3), (100000, 8), (250000, 6)]
     others = [(64, 64), (700, 700), (1024, 1024), (4096, 4096), (20000, 3), (20000, 8), (50000, 11), (8, 100000), (250000, 24),
-              (16384, 16384)]
+              (16384, 16384), (53, 400000)]
     kinds = [r[0] for r in shapes([f"plan {nx} {ny} 0" for nx, ny in one_wave + others])]
     assert kinds[:len(one_wave)] == [0] * len(one_wave)
     assert 0 not in kinds[len(one_wave):]
