@@ -66,6 +66,7 @@ extern "C" int sf_ctx_create(sf_ctx** out, int nx, int ny, void* stream)
     sf_ctx* c = new sf_ctx();
     c->nx = nx;
     c->ny = ny;
+    if (!markers_only) c->plan = pt_plan(nx, ny);
     c->stream = (hipStream_t)stream;
     hipError_t e = hipGetDevice(&c->device);
     // a marker-only context keeps 1-element placeholders for the grid scratch
@@ -252,7 +253,7 @@ static int ctx_pt_loop(sf_ctx* c, PTLoop* L, double* Vx_s, double* Vy_s, double*
     PTBuffers b{};
     const int rc = ctx_pt_buffers(c, fuse != 1, &b);
     if (rc) return rc;
-    L->init(b, fuse, rows, c->nx, c->ny, Vx_s, Vy_s, P, dVx, dVy);
+    L->init(b, fuse, rows, c->plan, c->nx, c->ny, Vx_s, Vy_s, P, dVx, dVy);
     L->tm = &c->timer;
     return SF_OK;
 }
@@ -481,7 +482,7 @@ int sf::solve_core(const SolveScratch& w, const char* who, double* P, double* Vx
     pp.max_nxy = k.max_nxy;
 
     PTLoop L;
-    L.init(w.pt, w.fuse, w.rows, nx, ny, Vx_s, Vy_s, P, dVx, dVy);
+    L.init(w.pt, w.fuse, w.rows, w.plan, nx, ny, Vx_s, Vy_s, P, dVx, dVy);
     L.tm = w.tm;
     L.pp = pp;
 
@@ -646,7 +647,7 @@ extern "C" int sf_solve_stokes(sf_ctx* c, double* P, double* Vx_pad, double* Vy_
     if (rc) return rc;
     const SolveScratch w{c->stream, b,       c->txx,    c->tyy,       c->txy, c->divv, c->rx,
                          c->ry,     c->part, c->scal,   c->hscal,     c->ev0, c->ev1,  c->seg,
-                         c->depth,  c->max_waves, fuse, rows,         &c->timer};
+                         c->depth,  c->max_waves, fuse, rows,         c->plan, &c->timer};
     return solve_core(w, "sf_solve_stokes", P, Vx_pad, Vy_pad, rho_vy, mu_b, mu_p, txx, tyy, txy, divV, dtauP, Rx,
                       Ry, dVx, dVy, dtauVx, dtauVy, Vx_s, Vy_s, g_y, dx, dy, nx, ny, dt, maxdisp, use_fss, eps,
                       iter_max, print_info, out);

@@ -178,8 +178,9 @@ struct PTLoop {
 
     // fuse: iterations per pass (0 size default, 1 one per launch, 2 to 4; larger values cap at 4);
     // pass_rows > 0 asks for the one-wave passes with that tile height
-    void init(const PTBuffers& buf, int fuse, int pass_rows, int nx_, int ny_, double* Vx_s, double* Vy_s, double* P,
-              double* dVx, double* dVy)
+    // size_plan: pt_plan(nx, ny)
+    void init(const PTBuffers& buf, int fuse, int pass_rows, const PTPlan& size_plan, int nx_, int ny_, double* Vx_s,
+              double* Vy_s, double* P, double* dVx, double* dVy)
     {
         nx = nx_;
         ny = ny_;
@@ -199,7 +200,7 @@ struct PTLoop {
         kmax = fuse == 0 ? pt_default_fusion(nx, ny) : std::min(fuse, 4);
         plan = PTPlan{};
         if (fuse == 0 && pass_rows == 0) {
-            plan = pt_plan(nx, ny);
+            plan = size_plan;
             if (plan.kind != PT_PLAN_NONE) kmax = plan.k;
         }
     }
@@ -225,6 +226,7 @@ struct SolveScratch {
     hipEvent_t ev0, ev1;                       // timing window; NULL: taken on the host clock
     int seg, depth, max_waves;                 // one-iteration kernel shape
     int fuse, rows;                            // iterations per pass and pass tile rows (0: defaults)
+    PTPlan plan;                               // pt_plan of the grid
     PassTimer* tm;                             // may be NULL
 };
 
@@ -283,6 +285,7 @@ struct sf_ctx {
     int seg = 0;        // rows per tile; 0 = size heuristic
     int depth = 0;      // rows of operands prefetched; 0 = size default
     int max_waves = -1; // 0 persistent (resident slots), > 0 cap, < 0 one wave per tile
+    sf::PTPlan plan{};  // pt_plan(nx, ny): some 10 us of host time on narrow grids, so once per context
     int fuse = 0;       // sf_ctx_set_pt_fusion: iterations / FP32 sweeps per pass (0 size default, 1..5)
     int pair_rows = 0;  // rows per tile of the multi-iteration passes; 0 = size default
     int fuse64 = 0;     // autotuner's choice for the FP64 passes only (0: none, then fuse / pair_rows apply; -1: the size default)

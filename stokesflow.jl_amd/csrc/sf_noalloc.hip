@@ -110,6 +110,7 @@ extern "C" int sf_solve_stokes_noalloc(void* hip_stream, double* P, double* Vx_p
     w.max_waves = -1;
     w.fuse = 0;
     w.rows = 0;
+    w.plan = pt_plan(nx, ny);
     w.tm = nullptr;
     return solve_core(w, who, P, Vx_pad, Vy_pad, rho_vy, mu_b, mu_p, txx, tyy, txy, divV, dtauP, Rx, Ry, dVx, dVy,
                       dtauVx, dtauVy, Vx_s, Vy_s, g_y, dx, dy, nx, ny, dt, maxdisp, use_fss, eps, iter_max,

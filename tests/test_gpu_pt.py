@@ -515,3 +515,30 @@ def test_autotune_replaces_explicit_passes(gpu):
         sfhip.time_passes(nx, ny, False)
         sfhip.set_pt_tuning(nx, ny, 0, 0, -1)
         sfhip.set_pt_fusion(nx, ny, 0, 0)
+
+
+def test_single_iteration_calls_cost_no_plan(gpu):
+    """Calls of one iteration on a narrow grid take as long with the size default as with one iteration
+    per launch asked for (1.4 times as long where every call worked the default out)."""
+    import time
+
+    nx, ny = 33, 4000
+    S = cases.smooth_state(nx, ny, seed=8)
+    G = to_gpu(S, STATE + ("rho_vy", "mu_b", "mu_p"))
+    best = {}
+    try:
+        for fuse in (0, 1):
+            sfhip.set_pt_fusion(nx, ny, fuse, 0)
+            times = []
+            for _ in range(8):
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(100):
+                    sfhip.pt_iterations(1, G["P"], G["Vx_s"], G["Vy_s"], G["dVx"], G["dVy"], G["rho_vy"], G["mu_b"],
+                                        G["mu_p"], 1.0, 1.0 / (nx - 1), 1.0 / (ny - 1), nx, ny, 0.01)
+                torch.cuda.synchronize()
+                times.append(time.perf_counter() - t0)
+            best[fuse] = min(times)
+    finally:
+        sfhip.set_pt_fusion(nx, ny, 0, 0)
+    assert best[0] < 1.2 * best[1], best
