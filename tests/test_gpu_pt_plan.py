@@ -71,3 +71,18 @@ def test_flat_grid_bitwise(gpu):
     finally:
         sfhip.time_passes(nx, ny, False)
     assert sorted((t["iters_per_launch"], t["launches"]) for t in launches) == [(3, 1), (4, 4)]
+
+
+@pytest.mark.parametrize("n_iter,passes", [(2, {}), (3, {2: 1}), (4, {2: 2}), (7, {3: 1, 4: 1}), (14, {7: 2}),
+                                           (15, {3: 1, 4: 3}), (21, {5: 3, 6: 1}), (28, {7: 4})])
+def test_resident_runs_end_in_the_callers_arrays(gpu, n_iter, passes):
+    """Runs of resident passes take an even number of launches (single iterations are not timed), so
+    nothing is copied back."""
+    nx, ny = 64, 64
+    sfhip.time_passes(nx, ny, True)
+    try:
+        _compare(cases.random_state(nx, ny, seed=n_iter), nx, ny, n_iter)
+        launches = {t["iters_per_launch"]: t["launches"] for t in sfhip.pass_times(nx, ny)}
+    finally:
+        sfhip.time_passes(nx, ny, False)
+    assert launches == passes
