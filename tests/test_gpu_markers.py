@@ -392,3 +392,27 @@ def test_materials_descriptor(gpu):
     rc = L.sf_marker_properties(ctx.handle, x.data_ptr(), y.data_ptr(), x.numel(), 0.0, 0.0, bad, 1, 1.0, 1.0,
                                 rho.data_ptr(), mu.data_ptr())
     assert rc == _lib.SF_ERR_ARG and b"unknown kind" in L.sf_last_error()
+
+
+@pytest.mark.parametrize("nm", [1, 36, 192, 193])
+def test_m2g_few_markers(gpu, nm):
+    """Up to 192 markers fit into one tile wherever they lie (here all in one cell), and the kernels
+    for tiles that do not fit are left out; from 193 on they run."""
+    from test_gpu_batch import kernel_launches
+
+    nx, ny = 20, 17
+    rng = np.random.default_rng(nm)
+    dx, dy = 1.0 / (nx - 1), 1.0 / (ny - 1)
+    x, y = (7.1 + 0.8 * rng.random(nm)) * dx, (5.1 + 0.8 * rng.random(nm)) * dy
+    val = 1.0 + rng.random(nm)
+    grid0 = np.asfortranarray(rng.random((nx, ny)))
+    out = []
+    n = kernel_launches(lambda: out.extend(m2g_gpu(0.0, 0.0, grid0, x, y, val, dx, dy, helper_shape=(nx, ny), helper_fill=3.0)),
+                        "m2g_far")
+    assert n == (0 if nm <= 192 else 2)
+    vg, (vws, ws), st = out
+    eg = grid0.copy(order="F")
+    evws, ews = O.zeros(nx, ny), O.zeros(nx, ny)
+    nb, ne = O.marker_to_grid(0.0, 0.0, eg, x, y, val, dx, dy, evws, ews)
+    assert np.array_equal(vg, eg) and np.array_equal(vws, evws) and np.array_equal(ws, ews)
+    assert (st["n_bad_markers"], st["n_empty_nodes"]) == (nb, ne)
