@@ -88,7 +88,8 @@ int sf_ctx_set_pt_tuning(sf_ctx *ctx, int rows, int depth, int max_waves);
  * passes cap it at 4); their default is 5 above 3072 nodes per side, else up to 12 by size, held
  * in registers.
  * rows: grid rows per tile of the pass (0 = size default; with rows alone, one-wave passes of a
- * default length).  Results are bit-identical either
+ * default length).  sf_pt_iterations runs of fewer than 14 iterations on grids whose default is
+ * the pipelined pass keep one-wave passes of up to 4.  Results are bit-identical either
  * way; the pass needs a second dVx/dVy buffer, allocated in the context on first use.  No
  * reference counterpart (the reference launches each of its kernels once per iteration). */
 int sf_ctx_set_pt_fusion(sf_ctx *ctx, int iters_per_launch, int rows);
@@ -240,8 +241,8 @@ int sf_solve_stokes_refined(sf_ctx *ctx, double *P, double *Vx_pad, double *Vy_p
  * take turns where their workgroups together number more than its CUs (two of more than about 100^2
  * nodes each), so they never hold each other up to that limit; processes that share a GPU know
  * nothing of each other and must not run them at the same time.
- * With precision 1 (WIDE only) every instance is solved as sf_solve_stokes_refined solves it,
- * with one launch per FP32 sweep of all active instances.
+ * With precision 1 (WIDE only) every instance is solved as sf_solve_stokes_refined solves it, a
+ * launch running several FP32 sweeps of all active instances.
  * In FP64 every PT iteration is bit-identical to sf_solve_stokes.  outs[i] gets instance i's dt_new,
  * err, niter, converged, dt_last (runtime = wall time of the batch).  No reference
  * counterpart (the reference solves one problem per process). */
@@ -257,7 +258,8 @@ typedef struct {
 
 enum { SF_BATCH_AUTO = 0, SF_BATCH_PERSISTENT = 1, SF_BATCH_WIDE = 2, SF_BATCH_GRID = 3 };
 typedef struct {
-    int rows;         /* grid rows per tile (<= 0: per instance, as the single solver's default) */
+    int rows;         /* grid rows per tile of the FP64 single iterations (<= 0: per instance, as the
+                         single solver's default); no effect with precision 1 */
     int depth;        /* wide: rows of operands prefetched, 1 or 2 (<= 0: 1); grid: PT iterations per
                          pass, 1 to 3 (<= 0: by size) */
     int threads;      /* persistent: threads per instance workgroup, multiple of 64, <= 512 (<= 0: 512) */
@@ -278,7 +280,8 @@ int sf_solve_stokes_batched(sf_ctx *ctx, const sf_batch_instance *inst, int n, c
  * takes the fastest (iterations per pass, rows) per size.  Each size's choice is then checked on
  * the whole batch -- every instance capped at 240 PT iterations, with the size defaults and with
  * the choice added -- and kept on the context only where the capped run is faster (one launch
- * mixes the sizes' tiles).  Copies of the caller's states are used (allocated and freed here;
+ * mixes the sizes' tiles).  The size defaults (planned over the whole set, sf_solve_stokes_batched)
+ * are not searched; a choice replaces them only where it beats them.  Copies of the caller's states are used (allocated and freed here;
  * the caller's arrays are not modified).  Later sf_solve_stokes_batched calls (wide mode) and
  * ensembles created from the context use the kept shapes; results do not depend on them.
  * table (may be NULL, table_cap entries) gets every candidate's time, n_table how many were

@@ -28,9 +28,10 @@
 // What bounds it: FP64 issue.  A row and stage takes 54 additions and multiplications, 6 to 10 DPP
 // moves and little else (77 VALU instructions against 126 in ptk_tile<4>, with 1.28 strip overlap
 // against 1.14 x 1.13), and seven iterations share one pass over memory (1.87 GB at 4096^2).  Measured
-// at 4096^2, us per iteration: 69.7 (ptk_tile<4> 108.6-112); 2048^2 19.4 (29.4); 1024^2 6.3 (9.0).  With
-// the barriers, the loads or the stores taken out a pass of 500 us took 457, 430 and 470, with all of
-// them out 383: the rest is arithmetic.  Two rows in flight in wave 0 did as well as three or four
+// at 4096^2, us per iteration: 64.0, 448 per pass (ptk_tile<4> 108.6-112); in the solver's loop 66 (109);
+// 2048^2 18.7 (28), 1024^2 6.4 (9.1).  With the barriers, the loads or the stores taken out a pass of
+// 500 us (before the short divisions and the wave priorities) took 457, 430 and 470, with all of them
+// out 383: the rest is arithmetic.  Two rows in flight in wave 0 did as well as three or four
 // (which spill); one stage per wave (more waves, shorter steps) was no faster, wave 0 being the
 // longest; three workgroups per CU fit (48 KB of LDS, 157 VGPRs) and want to be resident together:
 // a fourth round costs a whole one (pt_plan).

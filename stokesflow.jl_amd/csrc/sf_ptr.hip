@@ -71,7 +71,7 @@ static int64_t resident_tiles(int nx, int ny, int rows, int k)
 // per CU (up to L2- and MALL-sized grids; 0.58, 0.82, 1.06 from HBM, in the same proportions).
 //
 // Measured against the passes before (us per iteration): 64^2 1.30 (2.6), 301x257 1.64 (3.1), 512^2 2.6
-// (4.65), 700^2 3.85 (about 6.5) resident; 1024^2 6.3 (9.1), 2048^2 19.4 (29.4), 4096^2 69.7 (112)
+// (4.65), 700^2 3.85 (about 6.5) resident; 1024^2 6.3 (9.1), 2048^2 18.7 (28), 4096^2 64-66 (109)
 // pipelined.  They cross near 730^2: resident 800^2 5.3 against 4.7, pipelined 600^2 3.6 against 2.95.
 PTPlan pt_plan_resident(int nx, int ny, int kmax, double launch_us, double kept_us, double* us_per_iter)
 {

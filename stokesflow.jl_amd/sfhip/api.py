@@ -117,7 +117,8 @@ _contexts = {}
 def autotune_pt(nx, ny, iters=20, state=None, g_y=1.0, dx=None, dy=None):
     """Time every PT launch shape on an nx x ny grid (sf_ctx_autotune_pt) and keep the fastest
     for later solves of that size.  ``state`` (a :class:`FlowState`) gives the problem to time
-    on (copied, not modified); without it a synthetic problem is used.  Returns (best, table)."""
+    on (copied, not modified); without it a synthetic problem is used.  Returns (best, table); the entry
+    with ``iters_per_launch`` 0 is the size default's passes."""
     nx, ny = int(nx), int(ny)
     ctx = context(nx, ny)
     best = _lib.PTTuning()
