@@ -13,7 +13,7 @@ import sfhip
 from oracle import sf_oracle as O
 
 import cases
-from test_gpu_batch import OUT, kernel_launches, plume_instance, problem, single
+from test_gpu_batch import OUT, plume_instance, problem, single
 from test_gpu_ensemble import member, same
 
 pytestmark = pytest.mark.gpu
@@ -236,6 +236,8 @@ def test_grid_checks_of_narrow_grids(gpu):
                                             (900, 11, True), (4, 20000, True)])
 def test_grid_mode_flat_grids(gpu, nx, ny, resident):
     """Flat grids with more tiles than CUs take the one-wave passes."""
+    from test_gpu_batch import kernel_launches
+
     S = cases.smooth_state(nx, ny, seed=650)
     dx, dy = 1.0 / (nx - 1), 1.0 / (ny - 1)
     pb, G = problem(S, nx, ny, dx, dy, iterMax=47)
